@@ -193,20 +193,22 @@ int32_t mt_scene_destroy(mt_scene* scene);
 /* ------------------------------------------------------------------ */
 /* A. Traversal                                                       */
 /* ------------------------------------------------------------------ */
-#define MT_TRACE_PACKED 0    /* default: packed 64-B node / 48-B triangle layout,
-                                one ray per lane, short stack (= PACKED_STACK) */
+#define MT_TRACE_PACKED 0    /* default: packed 64-B node / 48-B triangle layout; plain batches
+                                as PACKED_STACK, the render's bounce queues as PACKED_POOL */
 #define MT_TRACE_REFERENCE 1 /* reads the reference's flat arrays directly */
 #define MT_TRACE_PACKED_NO_STACK 2 /* packed, one ray per lane, parent-link backtracking */
-#define MT_TRACE_PACKED_STACK 3    /* packed, one ray per lane, short stack */
-#define MT_TRACE_PACKED_REFILL 4   /* packed, short stack, persistent waves with refill */
+#define MT_TRACE_PACKED_STACK 3    /* packed, stack in LDS, each lane loads its own nodes
+                                      (coherent batches) */
+#define MT_TRACE_PACKED_REFILL 4   /* the same as PACKED_POOL */
 #define MT_TRACE_PACKED_SORTED 5   /* packed, short stack, each work-group's rays taken in
                                       direction-bin order (same results per ray) */
-#define MT_TRACE_PACKED_POOL 6     /* packed, short stack, each wave refills finished lanes
-                                      from its own run of 256 rays (same results per ray) */
+#define MT_TRACE_PACKED_POOL 6     /* packed, stack in LDS, nodes staged through LDS by the four
+                                      lanes of a quad together (incoherent batches; same
+                                      results per ray) */
 #define MT_TRACE_PACKED_BINNED 7   /* packed: the batch counting-sorted by origin cell
                                       (32^3 grid, Morton order) on the device, then traced
-                                      in that order by wave pools (same results per ray;
-                                      for incoherent batches) */
+                                      in that order as PACKED_POOL (same results per ray;
+                                      for large incoherent batches) */
 
 /* Closest hit (intersectMesh with bailout = false, NormalBVH.cl:14-92, as
  * run by IntersectPrimitives :94-123; launched at CDeviceGI.java:230 and
@@ -228,11 +230,11 @@ int32_t mt_trace_any(mt_context* ctx, const mt_scene* scene,
 
 /* Traversal autotuner (no counterpart in the reference, which has one
  * traversal kernel).  Every packed mode returns the same bits, but their
- * speed depends on the batch: one ray per lane with the short stack wins on
- * coherent rays, lane refill (persistent waves or wave pools) on incoherent
- * ones, ray binning on large incoherent ones.  Traces this batch (any = 0:
+ * speed depends on the batch: lanes that load their own nodes win on
+ * coherent rays, staged nodes on incoherent ones, ray binning on large
+ * incoherent ones.  Traces this batch (any = 0:
  * closest hit into prim/t; any != 0: any hit into occluded) with
- * MT_TRACE_PACKED_STACK, _REFILL, _POOL and _BINNED, `reps` timed runs each
+ * MT_TRACE_PACKED_STACK, _REFILL and _BINNED, `reps` timed runs each
  * after one warm-up, times them
  * with HIP events on the context stream and sets *best_mode to the fastest
  * and *best_ms to its mean time.  The outputs hold the batch's
@@ -704,14 +706,10 @@ int32_t mt_batch_set_iterations(mt_batch* batch, int32_t iterations);
  * Synchronises the context. */
 int32_t mt_batch_set_graphs(mt_batch* batch, int32_t on);
 /* Closest-hit traversal of the engine's shared queue (no counterpart in the
- * reference): MT_BATCH_TRACE_SPLIT (MT_TRACE_PACKED, the default: the
- * queue's front, the paths continuing from earlier bounces, with wave pools;
- * its back, the camera rays of newly started paths, one ray per lane),
- * MT_TRACE_PACKED_STACK (one ray per lane) or MT_TRACE_PACKED_POOL (wave
- * pools with lane refill; each lane loads its slot's scene).  Images do not
- * depend on it.  The choice the serving autotuner makes per workload
- * (multi-job workloads of 256 uneven jobs, and of Poisson arrivals: split
- * 64.0 jobs/s, one ray per lane 60.4, pools 59.8).  Synchronises the
+ * reference): MT_BATCH_TRACE_SPLIT (= MT_TRACE_PACKED, the default),
+ * MT_TRACE_PACKED_STACK or MT_TRACE_PACKED_POOL.  All of them run one kernel
+ * now (staged nodes; each lane takes its slot's scene with its ray); the call
+ * is kept for its callers.  Images do not depend on it.  Synchronises the
  * context. */
 #define MT_BATCH_TRACE_SPLIT 8
 int32_t mt_batch_set_trace_mode(mt_batch* batch, int32_t mode);

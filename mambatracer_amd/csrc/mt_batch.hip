@@ -273,7 +273,7 @@ __global__ __launch_bounds__(BT) void k_shade_jobs(ShadeJobsArgs A)
 // with the direct-light add fused in: an unoccluded entry adds its
 // contribution to its path's radiance in its job's buffer.  Work-group 0
 // adds the iteration's shadow rays to the running total.
-__global__ __launch_bounds__(BT) void k_shadow_jobs(const JobRec* __restrict__ jobs,
+__global__ __launch_bounds__(BT, WaveLds<WT_DIRECT>::WAVES) void k_shadow_jobs(const JobRec* __restrict__ jobs,
                                                     const MtSceneRef* __restrict__ refs,
                                                     const int* __restrict__ s_seg, int seg_cap,
                                                     const int2* __restrict__ s_tag, const float4* __restrict__ s_o,
@@ -281,26 +281,31 @@ __global__ __launch_bounds__(BT) void k_shadow_jobs(const JobRec* __restrict__ j
                                                     const float4* __restrict__ contrib,
                                                     unsigned long long* __restrict__ tot)
 {
-    const int k = seg_entry<JOB_SEGS>(seg_cap); // chunk-major: live chunks dispatch first
+    __shared__ WaveLds<WT_DIRECT> s_w[4];
     if (blockIdx.x == 0) {
         int c = 0;
         for (int p = threadIdx.x; p < JOB_SEGS; p += BT) c += s_seg[p];
         for (int o = 32; o > 0; o >>= 1) c += __shfl_xor(c, o);
         if (__lane_id() == 0 && c) atomicAdd(&tot[1], (unsigned long long)c);
     }
-    if (!seg_live<JOB_SEGS>(s_seg, seg_cap, k)) return;
-    const int2 tg = s_tag[k];
-    const int job = tg.x >> BOUNCE_BITS;
-    const MtSceneRef R = refs[job];
-    RayT r;
-    ray_init(r, s_o[k], s_d[k]);
-    int st[3] = {0, 0, 0};
-    int child = -1;
-    if (trace_packed<true, false, true>(R.pn, R.pt, R.root, r, child, st)) return;
-    const float4 c = contrib[k];
-    float4* L = jobs[job].L;
-    const float4 v = L[tg.y];
-    L[tg.y] = make_float4(v.x + c.x, v.y + c.y, v.z + c.z, v.w);
+    int next, end;
+    seg_run(s_seg, JOB_SEGS, seg_cap, WaveLds<WT_DIRECT>::SLOTS, next, end);
+    if (next >= end) return; // wave-uniform
+    wave_trace<true, true, WT_REFILL>(
+        s_w, refs[s_tag[next].x >> BOUNCE_BITS], next, end,
+        [&](int k, RayT& r, MtSceneRef& sc) {
+            sc = refs[s_tag[k].x >> BOUNCE_BITS];
+            ray_init(r, s_o[k], s_d[k]);
+        },
+        [&](bool fin, int k, float, int child, const MtSceneRef&) {
+            if (fin && child == WT_NONE) {
+                const int2 tg = s_tag[k];
+                const float4 c = contrib[k];
+                float4* L = jobs[tg.x >> BOUNCE_BITS].L;
+                const float4 v = L[tg.y];
+                L[tg.y] = make_float4(v.x + c.x, v.y + c.y, v.z + c.z, v.w);
+            }
+        });
 }
 
 } // namespace
@@ -344,7 +349,6 @@ struct mt_batch {
     int policy;
     int iters_per_step;       // wavefront iterations between host round trips
     int* nact;                // device: number of active jobs (read by the iteration kernels)
-    int trace_mode;           // closest hit: MT_BATCH_TRACE_SPLIT (default), MT_TRACE_PACKED_STACK or _POOL
     // The iterations of a step as one hipGraph per start parity of the queue
     // ping-pong: every size they use lives in device memory, so a capture
     // stays valid until the iterations per step change.
@@ -437,7 +441,7 @@ int32_t admit(mt_batch* b)
         rec.rr_start = d.render.rr_start;
         rec.flags = d.render.flags;
         rec.seed = d.render.seed;
-        MtSceneRef ref{d.scene->pnodes, d.scene->ptris, d.scene->root_ref, 0};
+        MtSceneRef ref{d.scene->pnodes, d.scene->ptris, d.scene->root_ref, d.scene->plain};
         k_set_job<<<1, DONE_SEGS, 0, b->ctx->stream>>>(b->jobs, b->refs, b->npaths, b->issued, b->done, b->done_tot,
                                                        b->cancel, b->max_jobs, J.slot, rec, ref);
         MT_LAUNCH_CHECK();
@@ -491,8 +495,7 @@ int32_t iterate(mt_batch* b)
                               b->gen_job, b->s_seg, b->tot);
     k_generate<<<grid, BT, 0, s>>>(b->jobs, b->cnt, b->gen_start, b->gen_pid0, b->gen_job, b->nact, q);
     MT_LAUNCH_CHECK();
-    int32_t rc = mt_trace_jobs(b->ctx, b->refs, &q.tag->x, BOUNCE_BITS, q.ro, q.rd, b->cnt + 1, Qc, b->prim,
-                               b->t, b->trace_mode, b->cnt); // cnt[0]: survivors, cnt[1]: survivors + new
+    int32_t rc = mt_trace_jobs(b->ctx, b->refs, &q.tag->x, BOUNCE_BITS, q.ro, q.rd, b->cnt + 1, Qc, b->prim, b->t);
     if (rc) return rc;
     ShadeJobsArgs A;
     A.jobs = b->jobs;
@@ -512,7 +515,7 @@ int32_t iterate(mt_batch* b)
     A.seg_cap = b->seg_cap;
     k_shade_jobs<<<grid, BT, 0, s>>>(A);
     MT_LAUNCH_CHECK();
-    k_shadow_jobs<<<mt_blocks((int64_t)JOB_SEGS * b->seg_cap, BT), BT, 0, s>>>(
+    k_shadow_jobs<<<JOB_SEGS * wave_seg_groups(b->seg_cap, JOB_SEGS, WaveLds<WT_DIRECT>::SLOTS), BT, 0, s>>>(
         b->jobs, b->refs, b->s_seg, b->seg_cap, b->s_tag, b->s_o, b->s_d, b->s_c, b->tot);
     MT_LAUNCH_CHECK();
     mt_payload P[4] = {{q.tag, nq.tag, 8}, {q.ro, nq.ro, 16}, {q.rd, nq.rd, 16}, {q.T, nq.T, 16}};
@@ -728,7 +731,6 @@ extern "C" int32_t mt_batch_create(mt_context* ctx, int32_t queue_capacity, uint
     b->policy = MT_BATCH_OLDEST_FIRST;
     b->iters_per_step = 1;
     b->use_graphs = true;
-    b->trace_mode = MT_BATCH_TRACE_SPLIT; // the serving autotuner's choice on both multi-job workloads
     for (int p = 0; p < 2; p++) {
         b->graph[p] = nullptr;
         b->gexec[p] = nullptr;
@@ -891,9 +893,7 @@ extern "C" int32_t mt_batch_set_trace_mode(mt_batch* b, int32_t mode)
     MT_ARG_CHECK(mode == MT_TRACE_PACKED || mode == MT_TRACE_PACKED_STACK || mode == MT_TRACE_PACKED_POOL ||
                      mode == MT_BATCH_TRACE_SPLIT,
                  "mt_batch_set_trace_mode: mode %d not supported by the batch engine", mode);
-    MT_HIP_CHECK(hipStreamSynchronize(b->ctx->stream)); // recorded graphs hold the old kernel
-    b->trace_mode = mode == MT_TRACE_PACKED ? MT_BATCH_TRACE_SPLIT : mode;
-    drop_graphs(b);
+    MT_HIP_CHECK(hipStreamSynchronize(b->ctx->stream)); // every mode runs the same kernel
     return MT_OK;
 }
 

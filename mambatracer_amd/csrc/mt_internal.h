@@ -80,8 +80,8 @@ struct mt_context {
 int32_t mt_ctx_side_stream(mt_context* ctx, hipStream_t* out);
 
 // Packed traversal layout derived from the reference arrays.
-//   node (64 B): float4 a = (L.min.xyz, L.max.x), b = (L.max.yz, R.min.xy),
-//                float4 c = (R.min.z, R.max.xyz), int4 d = (left, right, parent, sibling)
+//   node (64 B): per axis float4 (L.min, R.min, L.max, R.max), then
+//                int4 (left, right, parent, sibling)
 //   refs: >= 0 interior node (packed index), < 0 leaf ~rank
 //   tri  (48 B): float4 (p1.xyz, e1.x), (e1.yz, e2.xy), (e2.z, prim bits, parent, sibling)
 struct mt_scene {
@@ -92,6 +92,7 @@ struct mt_scene {
     float4* pnodes;        // [max(num_interior,1) * 4]
     float4* ptris;         // [num_tris * 3]
     int32_t root_ref;      // 0, or ~0 when the tree is a single leaf
+    int32_t plain;         // every box is finite (|x| <= 1e30) and not inverted
 };
 
 struct mt_lightgrid {
@@ -148,7 +149,7 @@ struct MtSceneRef {
     const float4* pn;
     const float4* pt;
     int32_t root;
-    int32_t pad;
+    int32_t plain; // mt_scene::plain
 };
 
 // A queue split into nseg segments of seg_cap entries; segment p holds
@@ -165,11 +166,9 @@ struct MtSegQueue {
 
 // Closest hit (prim, t) over a queue that mixes jobs: slot i's scene is
 // refs[tag[2*i] >> shift]; entries i < *d_count (clamped to capacity).
-// mode MT_BATCH_TRACE_SPLIT: entries below *d_split (the earlier bounces'
-// survivors) with wave pools, the rest (new camera rays) one ray per lane.
 int32_t mt_trace_jobs(mt_context* ctx, const MtSceneRef* refs, const int32_t* tag, int32_t shift,
                       const float4* o_tmin, const float4* d_tmax, const int32_t* d_count, int32_t capacity,
-                      int32_t* prim, float* t, int32_t mode, const int32_t* d_split);
+                      int32_t* prim, float* t);
 // Any hit over a segmented queue for one scene (traversal mode as
 // mt_trace_any; the per-lane refill mode traverses like the short-stack mode
 // here); stats as mt_trace_any, indexed by queue entry.

@@ -67,51 +67,36 @@ __global__ __launch_bounds__(RT) void k_camera(Camera C, int npaths, const uint3
 
 // Bounce 0 of the fused loop: path pid = slot traces its camera ray
 // (generated here, never stored) to its closest hit; same per-ray traversal
-// as mt_trace_closest's default mode, so prim/t are the same bits.  POOL 0:
-// one path per lane, work-groups renumbered in per-XCD runs
-// (xcd_chunked_group); POOL > 0: each wave traces the run of 64 * POOL
-// consecutive paths (4 runs per work-group), refilling finished lanes
-// (pool_trace).
-template <int POOL>
-__global__ __launch_bounds__(RT) void k_trace_camera(Camera C, int npaths, const uint32_t* __restrict__ d_seed,
-                                                     const float4* __restrict__ pn, const float4* __restrict__ pt,
-                                                     int root, int* __restrict__ prim, float* __restrict__ tout,
-                                                     int* __restrict__ count0)
+// as mt_trace_closest, so prim/t are the same bits.  Each wave traces the run
+// of `run` consecutive paths, refilling finished lanes (wave_trace);
+// work-groups in per-XCD runs (a compact patch of pixels).
+template <bool WIDE>
+__global__ __launch_bounds__(RT, WaveLds<WT_DIRECT>::WAVES) void k_trace_camera(
+    Camera C, int npaths, int run, const uint32_t* __restrict__ d_seed, MtSceneRef scene, int* __restrict__ prim,
+    float* __restrict__ tout, int* __restrict__ count0)
 {
+    __shared__ WaveLds<WT_DIRECT> s_w[4];
     if (blockIdx.x == 0 && threadIdx.x == 0) *count0 = npaths;
     const uint32_t seed = *d_seed;
-    if (POOL > 0) {
-        const int next = (int)(blockIdx.x * 4 + (threadIdx.x >> 6)) * (64 * POOL);
-        const int end = npaths < next + 64 * POOL ? npaths : next + 64 * POOL;
-        if (next >= end) return;
-        const Camera Cr = C; // a register copy: a reference into the kernel argument spills it to scratch
-        pool_trace<false>(
-            pn, pt, root, next, end,
-            [&](int pid, RayT& r, const float4*&, const float4*&, int&) {
-                float4 o, d;
-                camera_ray(Cr, pid, seed, o, d);
-                ray_init(r, o, d);
-            },
-            [&](bool fin, int pid, const RayT& r, const TravState& S) {
-                if (fin) {
-                    prim[pid] = S.hit ? S.child : -1;
-                    tout[pid] = r.tmax;
-                }
-            });
-        return;
-    }
-    // work-groups in per-XCD runs (16K paths, a compact patch of pixels)
-    const int pid = (int)xcd_chunked_group(blockIdx.x, gridDim.x, XCD_RUN) * (int)blockDim.x + (int)threadIdx.x;
-    if (pid >= npaths) return;
-    float4 o, d;
-    camera_ray(C, pid, seed, o, d);
-    RayT r;
-    ray_init(r, o, d);
-    int st[3] = {0, 0, 0};
-    int child = -1;
-    const int h = trace_packed<false, false, true>(pn, pt, root, r, child, st);
-    prim[pid] = h ? child : -1;
-    tout[pid] = r.tmax;
+    const unsigned g = xcd_chunked_group(blockIdx.x, gridDim.x, XCD_RUN);
+    const int64_t first = ((int64_t)g * 4 + (threadIdx.x >> 6)) * run;
+    if (first >= npaths) return;
+    const int next = (int)first;
+    const int end = npaths - next < run ? npaths : next + run;
+    const Camera Cr = C; // a register copy: a reference into the kernel argument spills it to scratch
+    wave_trace<false, WIDE, WT_REFILL_CAMERA>(
+        s_w, scene, next, end,
+        [&](int pid, RayT& r, MtSceneRef&) {
+            float4 o, d;
+            camera_ray(Cr, pid, seed, o, d);
+            ray_init(r, o, d);
+        },
+        [&](bool fin, int pid, float t, int child, const MtSceneRef&) {
+            if (fin) {
+                prim[pid] = leaf_prim(scene.pt, child);
+                tout[pid] = t;
+            }
+        });
 }
 
 // Any hit over the segmented shadow queue with the direct-light add fused
@@ -120,57 +105,22 @@ __global__ __launch_bounds__(RT) void k_trace_camera(Camera C, int npaths, const
 // With the light-grid guided environment (pend != nullptr), an unoccluded
 // environment sample also adds its luminance to its grid entry (s_lg: entry,
 // luminance bits; the commented-out accumLightGrid, Render.cl:458-459).
-// POOL 0: one entry per lane; POOL > 0: each wave traces a run of 64 * POOL
-// entries of one segment, refilling finished lanes (pool_trace).
-template <int POOL>
-__global__ __launch_bounds__(RT) void k_trace_shadow(const float4* __restrict__ pn, const float4* __restrict__ pt,
-                                                     int root, const int* __restrict__ seg_counts, int seg_cap,
-                                                     const float4* __restrict__ s_o, const float4* __restrict__ s_d,
-                                                     const float4* __restrict__ contrib, const int* __restrict__ queue,
-                                                     float4* __restrict__ L, const int2* __restrict__ s_lg,
-                                                     unsigned long long* __restrict__ pend)
+// Each wave traces its share of one segment, refilling finished lanes.
+template <bool WIDE>
+__global__ __launch_bounds__(RT, WaveLds<WT_DIRECT>::WAVES) void k_trace_shadow(
+    MtSceneRef scene, const int* __restrict__ seg_counts, int seg_cap, const float4* __restrict__ s_o,
+    const float4* __restrict__ s_d, const float4* __restrict__ contrib, const int* __restrict__ queue,
+    float4* __restrict__ L, const int2* __restrict__ s_lg, unsigned long long* __restrict__ pend)
 {
-    if (POOL > 0) {
-        int next, end;
-        pool_seg_run(seg_counts, SHADOW_SEGS, seg_cap, 64 * POOL, next, end);
-        if (next >= end) return; // wave-uniform
-        pool_trace<true>(
-            pn, pt, root, next, end,
-            [&](int k, RayT& r, const float4*&, const float4*&, int&) { ray_init(r, s_o[k], s_d[k]); },
-            [&](bool fin, int k, const RayT&, const TravState& S) {
-                const bool vis = fin && !S.hit;
-                if (vis) {
-                    const float4 c = contrib[k];
-                    const int slot = __float_as_int(c.w);
-                    const int pid = queue ? queue[slot] : slot;
-                    const float4 v = L[pid];
-                    L[pid] = make_float4(v.x + c.x, v.y + c.y, v.z + c.z, v.w);
-                }
-                if (pend) { // the whole wave is active here
-                    int2 e = make_int2(-1, 0);
-                    if (vis) e = s_lg[k];
-                    lg_wave_accum(e.x >= 0, e.x, lg_fixed(__int_as_float(e.y)), pend);
-                }
-            });
-        return;
-    }
-    // segment sweep (SEG_SWEEP groups per segment): one entry per lane per chunk
-    const unsigned v = seg_sweep_group();
-    const int p = (int)(v % SHADOW_SEGS);
-    int cnt = seg_counts[p];
-    cnt = cnt < seg_cap ? cnt : seg_cap;
-    const int stride = (int)(gridDim.x / SHADOW_SEGS) * (int)blockDim.x;
-    for (int off = (int)(v / SHADOW_SEGS) * (int)blockDim.x; off < cnt; off += stride) {
-        const int k = p * seg_cap + off + (int)threadIdx.x;
-        const bool live = off + (int)threadIdx.x < cnt;
-        if (__ballot(live) == 0ull) continue; // wave-uniform
-        bool vis = false;
-        if (live) {
-            RayT r;
-            ray_init(r, s_o[k], s_d[k]);
-            int st[3] = {0, 0, 0};
-            int child = -1;
-            vis = !trace_packed<true, false, true>(pn, pt, root, r, child, st);
+    __shared__ WaveLds<WT_DIRECT> s_w[4];
+    int next, end;
+    seg_run(seg_counts, SHADOW_SEGS, seg_cap, WaveLds<WT_DIRECT>::SLOTS, next, end);
+    if (next >= end) return; // wave-uniform
+    wave_trace<true, WIDE, WT_REFILL_ANY>(
+        s_w, scene, next, end,
+        [&](int k, RayT& r, MtSceneRef&) { ray_init(r, s_o[k], s_d[k]); },
+        [&](bool fin, int k, float, int child, const MtSceneRef&) {
+            const bool vis = fin && child == WT_NONE;
             if (vis) {
                 const float4 c = contrib[k];
                 const int slot = __float_as_int(c.w);
@@ -178,13 +128,12 @@ __global__ __launch_bounds__(RT) void k_trace_shadow(const float4* __restrict__ 
                 const float4 v = L[pid];
                 L[pid] = make_float4(v.x + c.x, v.y + c.y, v.z + c.z, v.w);
             }
-        }
-        if (pend) { // the whole wave is active here
-            int2 e = make_int2(-1, 0);
-            if (vis) e = s_lg[k];
-            lg_wave_accum(e.x >= 0, e.x, lg_fixed(__int_as_float(e.y)), pend);
-        }
-    }
+            if (pend) { // the whole wave is active here
+                int2 e = make_int2(-1, 0);
+                if (vis) e = s_lg[k];
+                lg_wave_accum(e.x >= 0, e.x, lg_fixed(__int_as_float(e.y)), pend);
+            }
+        });
 }
 
 struct ShadeArgs {
@@ -534,7 +483,6 @@ struct RenderPlan {
         oIlp, oTot, oSeed, oSlg, oHit, oHsc, oTail;
     mt_lightgrid* grid; // guided environment mode: the grid the render samples and accumulates into
     bool fused; // camera rays traced in place, shadow adds fused, next queue appended by the shading stage
-    bool pool;  // fused kernels trace wave runs with lane refill (pool_trace)
     int tail;   // fused loop: bounces tail..nb-1 run in one k_tail launch (0: none)
     bool borrowed; // base is the context's reusable workspace (mt_render), not owned
     hipEvent_t ev[4 * 64];
@@ -625,7 +573,6 @@ int32_t plan_render(const mt_scene* scene, const float* materials, const mt_envm
     R.want_ilp = (desc->flags & MT_RENDER_TRAVERSAL_STATS) != 0;
     R.fused = (desc->mode == MT_TRACE_PACKED || desc->mode == MT_TRACE_PACKED_STACK ||
                desc->mode == MT_TRACE_PACKED_SORTED || desc->mode == MT_TRACE_PACKED_POOL) && !R.want_ilp;
-    R.pool = desc->mode == MT_TRACE_PACKED_POOL;
     R.tail = (desc->flags >> MT_RENDER_TAIL_SHIFT) & 63;
     if (!R.fused || R.tail >= R.nb) R.tail = 0; // the tail applies to the fused loop's bounces >= 1
     R.profile = (desc->flags & MT_RENDER_PROFILE) != 0;
@@ -727,10 +674,11 @@ int32_t enqueue_render(mt_context* ctx, RenderPlan& R)
     const int seg_chunks = (int)(((int64_t)seg_cap + RT - 1) / RT);
     const int gsweep = SHADOW_SEGS * (seg_chunks < SEG_SWEEP ? seg_chunks : SEG_SWEEP);
     const int gtail = SHADOW_SEGS * (seg_chunks < TAIL_SWEEP ? seg_chunks : TAIL_SWEEP);
-    // wave-pool kernels: runs of 64 * POOL_RAYS entries, 4 per work-group
-    const int64_t pool_group = 4 * 64 * (int64_t)POOL_RAYS;
-    const int gcam_pool = mt_blocks(np, (int)pool_group);
-    const int gshadow_pool = SHADOW_SEGS * (int)((seg_cap + pool_group - 1) / pool_group);
+    const MtSceneRef sref{scene->pnodes, scene->ptris, scene->root_ref, scene->plain};
+    const bool wide = scene_wide(scene);
+    const int cam_run = wave_run(np, WaveLds<WT_DIRECT>::SLOTS);
+    const int gcam = mt_blocks(np, 4 * cam_run);
+    const int gany = SHADOW_SEGS * wave_seg_groups(seg_cap, SHADOW_SEGS, WaveLds<WT_DIRECT>::SLOTS);
     unsigned long long* tot = reinterpret_cast<unsigned long long*>(base + R.oTot);
     int* ilp = R.want_ilp ? I(R.oIlp) : nullptr;
     hipEvent_t* ev = R.ev;
@@ -822,14 +770,9 @@ int32_t enqueue_render(mt_context* ctx, RenderPlan& R)
         }
         if (profile && (rc = mark(ev[4 * b]))) break;
         if (first) {
-            if (R.pool)
-                k_trace_camera<POOL_RAYS><<<gcam_pool, RT, 0, st>>>(R.C, np, seed_ptr(R), scene->pnodes, scene->ptris,
-                                                                    scene->root_ref, I(R.oPrim),
-                                                                    reinterpret_cast<float*>(base + R.oT_), counts);
-            else
-                k_trace_camera<0><<<grid, RT, 0, st>>>(R.C, np, seed_ptr(R), scene->pnodes, scene->ptris,
-                                                       scene->root_ref, I(R.oPrim),
-                                                       reinterpret_cast<float*>(base + R.oT_), counts);
+            auto kern = wide ? k_trace_camera<true> : k_trace_camera<false>;
+            kern<<<gcam, RT, 0, st>>>(R.C, np, cam_run, seed_ptr(R), sref, I(R.oPrim),
+                                      reinterpret_cast<float*>(base + R.oT_), counts);
             rc = chk();
         } else if (fused) {
             rc = mt_trace_closest_seg(ctx, scene, ro[cur], rd[cur], MtSegQueue{qsc + (size_t)b * SHADOW_SEGS,
@@ -868,14 +811,9 @@ int32_t enqueue_render(mt_context* ctx, RenderPlan& R)
                 }
                 ss = R.side;
             }
-            if (R.pool)
-                k_trace_shadow<POOL_RAYS><<<gshadow_pool, RT, 0, ss>>>(
-                    scene->pnodes, scene->ptris, scene->root_ref, seg_counts, seg_cap, F4(R.oSo), F4(R.oSd),
-                    F4(R.oSc), first ? nullptr : q[cur], S.L, A.s_lg, R.grid ? R.grid->pend : nullptr);
-            else
-                k_trace_shadow<0><<<gsweep, RT, 0, ss>>>(
-                    scene->pnodes, scene->ptris, scene->root_ref, seg_counts, seg_cap, F4(R.oSo), F4(R.oSd),
-                    F4(R.oSc), first ? nullptr : q[cur], S.L, A.s_lg, R.grid ? R.grid->pend : nullptr);
+            auto kern = wide ? k_trace_shadow<true> : k_trace_shadow<false>;
+            kern<<<gany, RT, 0, ss>>>(sref, seg_counts, seg_cap, F4(R.oSo), F4(R.oSd), F4(R.oSc),
+                                      first ? nullptr : q[cur], S.L, A.s_lg, R.grid ? R.grid->pend : nullptr);
             if ((rc = chk())) break;
             if (overlap) {
                 const hipError_t x = hipEventRecord(R.join[b], R.side);

@@ -16,12 +16,16 @@
 //  * MT_TRACE_REFERENCE reads the reference's flat arrays (7-int nodes,
 //    8-float boxes, 10-int faces, float4 points) as IntersectPrimitives does.
 //  * MT_TRACE_PACKED (default) reads a layout derived once per scene: each
-//    interior node is one 64-byte record holding both child boxes, both child
-//    references and its own parent/sibling; each leaf triangle is one 48-byte
-//    record (p1, e1 = p2 - p1, e2 = p3 - p1, primitive id, and the leaf's
-//    parent/sibling in its two spare words) stored in leaf order.  e1/e2 are the same float subtractions the reference performs
-//    per test, so every intersection rounds identically.  An interior step
-//    fetches 64 B instead of 148 B, a leaf 48 B instead of 116 B.
+//    interior node is one 64-byte record holding both child boxes, grouped by axis
+//    ({L.min, R.min, L.max, R.max} x, y, z), both child references and its own
+//    parent/sibling; each leaf triangle is one 48-byte record (p1, e1 = p2 - p1,
+//    e2 = p3 - p1, primitive id, and the leaf's parent/sibling in its two spare
+//    words) stored in leaf order.  e1/e2 are the same float subtractions the
+//    reference performs per test, so every intersection rounds identically.  An
+//    interior step fetches 64 B instead of 148 B, a leaf 48 B instead of 116 B.
+// Rays of the packed layout are traced by wave_trace (mt_traverse.h); the
+// reference layout, the walk without a stack, the direction-sorted lanes and
+// the counting runs take one ray per lane (k_trace, k_trace_sorted).
 #include "mt_traverse.h"
 
 #include <cstdio>
@@ -44,7 +48,8 @@ struct TraceArgs {
     float* tout;
     int* occluded;
     int* stats;
-    unsigned* ctr; // refill kernel: [0] next ray, [1] waves finished; zero between launches
+    int plain;    // mt_scene::plain
+    int run;      // rays per wave over a plain queue
     MtSegQueue seg; // segmented queue (seg.counts set) instead of *d_count
     const int* order; // binned traversal: entry k is ray order[k], its results go there (null: ray k)
 };
@@ -75,105 +80,9 @@ __device__ __forceinline__ int queue_entry(const TraceArgs& A)
     return blockIdx.x * blockDim.x + threadIdx.x;
 }
 
-template <bool ANY, bool STATS, class State>
-__device__ __forceinline__ void store_result(const TraceArgs& A, int id, const RayT& r, const State& S)
-{
-    if (A.order) id = A.order[id];
-    if (ANY) {
-        A.occluded[id] = S.hit;
-    } else {
-        A.prim[id] = S.hit ? S.child : -1;
-        A.tout[id] = r.tmax;
-    }
-    if (STATS) {
-        A.stats[3 * id + 0] = S.st[0];
-        A.stats[3 * id + 1] = S.st[1];
-        A.stats[3 * id + 2] = S.st[2];
-    }
-}
-
-// Persistent traversal with per-lane ray refill.  Incoherent rays differ a
-// lot in length, and a wave that owns 64 rays runs until its longest one
-// ends.  Here a wave takes chunks of REFILL_CHUNK consecutive rays with one
-// global atomic and, whenever at least REFILL_MIN of its lanes have finished
-// (or all have), hands the chunk's next rays to the idle lanes (ballot +
-// mbcnt), so lanes stay busy until the rays run out.  Each ray is traversed
-// by trace_packed_step in the reference's visiting order; only the mapping of
-// rays to lanes changes.  The last wave to leave clears the counters.
-constexpr int REFILL_CHUNK = 1024;
-constexpr int REFILL_MIN = 16;
-
-template <bool ANY, bool STATS>
-__global__ __launch_bounds__(256) void k_trace_refill(TraceArgs A)
-{
-    int count = *A.d_count;
-    if (count > A.capacity) count = A.capacity;
-    const int lane = __lane_id();
-    int cnext = 0, cend = 0; // wave-uniform chunk cursor
-    bool drained = false;    // wave-uniform: the global counter is past count
-    bool active = false;
-    int id = 0;
-    RayT r;
-    TravState S;
-    for (;;) {
-        uint64_t idle = __ballot(!active);
-        if (idle && !drained && (idle == ~0ull || __popcll(idle) >= REFILL_MIN)) {
-            uint64_t want = idle;
-            while (want) {
-                if (cnext >= cend) {
-                    unsigned base = 0;
-                    if (lane == 0) base = atomicAdd(&A.ctr[0], (unsigned)REFILL_CHUNK);
-                    base = __shfl(base, 0);
-                    if (base >= (unsigned)count) {
-                        drained = true;
-                        break;
-                    }
-                    cnext = (int)base;
-                    cend = (int)base + REFILL_CHUNK < count ? (int)base + REFILL_CHUNK : count;
-                }
-                int take = cend - cnext;
-                int n = __popcll(want);
-                take = take < n ? take : n;
-                bool got = false;
-                if ((want >> lane) & 1ull) {
-                    int rk = (int)lane_rank(want);
-                    if (rk < take) {
-                        id = cnext + rk;
-                        const int src = A.order ? A.order[id] : id;
-                        ray_init(r, A.o_tmin[src], A.d_tmax[src]);
-                        S.init(A.root);
-                        active = true;
-                        got = true;
-                    }
-                }
-                cnext += take;
-                want &= ~__ballot(got);
-            }
-        }
-        if (!__any(active)) {
-            if (drained) break;
-            continue;
-        }
-        if (active && trace_packed_step<ANY, STATS, true>(A.pn, A.pt, r, S)) {
-            store_result<ANY, STATS>(A, id, r, S);
-            active = false;
-        }
-    }
-    if (lane == 0) {
-        unsigned waves = gridDim.x * (blockDim.x >> 6);
-        unsigned done = atomicAdd(&A.ctr[1], 1u);
-        if (done == waves - 1) {
-            atomicExch(&A.ctr[0], 0u);
-            atomicExch(&A.ctr[1], 0u);
-        }
-    }
-}
-
-// One ray per lane over a capacity-sized grid; slots >= *d_count exit at
-// once (the hardware dispatcher retires such work-groups in microseconds,
-// cheaper than a persistent grid drawing rays from one global counter).
-// LAYOUT: 0 packed + short stack, 1 reference arrays, 2 packed without the
-// short stack (the reference's parent-link pops, kept for comparison).
+// One ray per lane over a capacity-sized grid; slots >= *d_count exit at once.
+// LAYOUT: 0 packed + short stack (counting runs), 1 reference arrays, 2 packed
+// without the short stack (the reference's parent-link pops).
 template <bool ANY, bool STATS, int LAYOUT>
 __global__ __launch_bounds__(256) void k_trace(TraceArgs A)
 {
@@ -199,18 +108,17 @@ __global__ __launch_bounds__(256) void k_trace(TraceArgs A)
     }
 }
 
-// Wave-pool traversal (pool_trace): each wave owns a run of 64 * POOL
-// consecutive queue entries (segmented queue: work-group b takes chunk
-// b / nseg of segment b % nseg, 256 * POOL entries, one run per wave; over a
+// Wave traversal (wave_trace) of a queue: each wave owns a run of consecutive
+// entries (segmented queue: an even share of its segment, seg_run; over a
 // binned order, work-groups in per-XCD runs) and refills its finished lanes
 // from it.
-template <bool ANY, int POOL, int SS = MT_SHORT_STACK>
-__global__ __launch_bounds__(256) void k_trace_pool(TraceArgs A)
+template <bool ANY, bool WIDE, WaveForm F>
+__global__ __launch_bounds__(256, WaveLds<F>::WAVES) void k_trace_wave(TraceArgs A)
 {
-    constexpr int RUN = 64 * POOL;
+    __shared__ WaveLds<F> s_w[4];
     int next, end;
     if (A.seg.counts) {
-        pool_seg_run(A.seg.counts, A.seg.nseg, A.seg.seg_cap, RUN, next, end);
+        seg_run(A.seg.counts, A.seg.nseg, A.seg.seg_cap, WaveLds<F>::SLOTS, next, end);
     } else {
         int count = *A.d_count;
         count = count < A.capacity ? count : A.capacity;
@@ -219,20 +127,30 @@ __global__ __launch_bounds__(256) void k_trace_pool(TraceArgs A)
         // walk the same subtrees: the groups that hold entries are numbered
         // in per-XCD runs (the grid is sized for the capacity; the rest leave
         // at once below)
-        const unsigned used = (unsigned)(((int64_t)count + 4 * RUN - 1) / (4 * RUN));
+        const unsigned used = (unsigned)(((int64_t)count + 4 * A.run - 1) / (4 * A.run));
         const unsigned g = A.order && blockIdx.x < used ? xcd_chunked_group(blockIdx.x, used, XCD_RUN) : blockIdx.x;
-        next = (int)(g * 4 + (threadIdx.x >> 6)) * RUN;
-        end = count < next + RUN ? count : next + RUN;
+        const int64_t first = ((int64_t)g * 4 + (threadIdx.x >> 6)) * A.run;
+        if (first >= count) return;
+        next = (int)first;
+        end = count - next < A.run ? count : next + A.run;
     }
     if (next >= end) return;
-    pool_trace<ANY, SS>(
-        A.pn, A.pt, A.root, next, end,
-        [&](int id, RayT& r, const float4*&, const float4*&, int&) {
+    wave_trace<ANY, WIDE, WT_REFILL>(
+        s_w, MtSceneRef{A.pn, A.pt, A.root, A.plain}, next, end,
+        [&](int id, RayT& r, MtSceneRef&) {
             const int src = A.order ? A.order[id] : id; // binned: entry id is ray order[id]
             ray_init(r, A.o_tmin[src], A.d_tmax[src]);
         },
-        [&](bool fin, int id, const RayT& r, const TravStateN<SS>& S) {
-            if (fin) store_result<ANY, false>(A, id, r, S);
+        [&](bool fin, int id, float t, int child, const MtSceneRef&) {
+            if (fin) {
+                const int dst = A.order ? A.order[id] : id;
+                if (ANY) {
+                    A.occluded[dst] = child != WT_NONE;
+                } else {
+                    A.prim[dst] = leaf_prim(A.pt, child);
+                    A.tout[dst] = t;
+                }
+            }
         });
 }
 
@@ -307,22 +225,31 @@ __global__ __launch_bounds__(256) void k_trace_sorted(TraceArgs A)
 }
 
 // Rays of many jobs in one queue: ray id's scene is refs[tag[2*id] >> shift]
-// (the job word of a wavefront slot).  Same per-ray traversal as k_trace
-// LAYOUT 0, so a ray's result does not depend on which queue carries it.
-__global__ __launch_bounds__(256) void k_trace_jobs(const MtSceneRef* __restrict__ refs, const int* __restrict__ tag,
-                                                    int shift, TraceArgs A, const int* __restrict__ first)
+// (the job word of a wavefront slot); a lane takes its ray's scene with the
+// ray, so a ray's result does not depend on which queue carries it.
+// Staged: 24 uneven soup jobs 23.4 -> 15.4 ms (direct 17.0).
+__global__ __launch_bounds__(256, WaveLds<WT_STAGED>::WAVES) void k_trace_jobs(const MtSceneRef* __restrict__ refs,
+                                                                              const int* __restrict__ tag, int shift,
+                                                                              TraceArgs A)
 {
-    // first != nullptr: the entries from *first on (grid sized for all)
-    const int id = (first ? *first : 0) + (int)(blockIdx.x * blockDim.x + threadIdx.x);
-    if (!entry_live(A, id)) return;
-    const MtSceneRef R = refs[tag[2 * id] >> shift];
-    RayT r;
-    ray_init(r, A.o_tmin[id], A.d_tmax[id]);
-    int st[3];
-    int child = -1;
-    int h = trace_packed<false, false, true>(R.pn, R.pt, R.root, r, child, st);
-    A.prim[id] = h ? child : -1;
-    A.tout[id] = r.tmax;
+    __shared__ WaveLds<WT_STAGED> s_w[4];
+    int count = *A.d_count;
+    count = count < A.capacity ? count : A.capacity;
+    const int next = (int)(blockIdx.x * 4 + (threadIdx.x >> 6)) * A.run;
+    const int end = count < next + A.run ? count : next + A.run;
+    if (next >= end) return;
+    wave_trace<false, true, WT_REFILL>(
+        s_w, refs[tag[2 * next] >> shift], next, end,
+        [&](int id, RayT& r, MtSceneRef& sc) {
+            sc = refs[tag[2 * id] >> shift];
+            ray_init(r, A.o_tmin[id], A.d_tmax[id]);
+        },
+        [&](bool fin, int id, float t, int child, const MtSceneRef& sc) {
+            if (fin) {
+                A.prim[id] = leaf_prim(sc.pt, child);
+                A.tout[id] = t;
+            }
+        });
 }
 
 // ---------------------------------------------------------------- binned traversal
@@ -333,12 +260,12 @@ __global__ __launch_bounds__(256) void k_trace_jobs(const MtSceneRef* __restrict
 // scene's root box (Morton order), with a one-pass counting sort (per-tile
 // histograms in LDS, an exclusive scan of the bin-major tile x bin matrix,
 // a scatter of the ray indices in key order), then traces the rays in that
-// order with wave pools (k_trace_pool), each result stored at the ray's own index.
+// order (k_trace_wave), each result stored at the ray's own index.
 // Rays that start near each other visit much the same upper nodes while they
 // are in flight together.  Per-ray results are those of any other mode.
-// (64M random rays through 4M triangles, closest / any hit: 8^3 cells x
-// direction octant 66.0 / 41.1 ms, 16^3 cells 63.8 / 39.0, 32^3 cells
-// 63.5 / 38.6; 4^3 cells x 64 direction bins 67.3 / 41.3.)
+// (64M random rays through 4M triangles, closest / any hit, measured with an
+// earlier traversal: 8^3 cells x direction octant 66.0 / 41.1 ms, 16^3 cells
+// 63.8 / 39.0, 32^3 cells 63.5 / 38.6; 4^3 cells x 64 direction bins 67.3 / 41.3.)
 constexpr int BIN_CELL_BITS = 5;                // cells per axis: 2^BIN_CELL_BITS
 constexpr int BIN_CELLS = 1 << BIN_CELL_BITS;
 constexpr int BIN_COUNT = 1 << (3 * BIN_CELL_BITS); // keys fit the 16-bit key array; LDS: 128 KB per group
@@ -356,7 +283,6 @@ constexpr int BIN_TILES_TARGET = 256;
 // store latency (64M rays: sort 2.7 ms per stage with 256 threads, step
 // 86.8 -> 85.5 ms with 1024)
 constexpr int BIN_THREADS = 1024;
-constexpr int BINNED_POOL_RAYS = 8; // rays per lane of a wave's run when tracing the sorted order
 
 __device__ __forceinline__ int bin_axis(float o, float lo, float scale)
 {
@@ -434,31 +360,6 @@ __global__ __launch_bounds__(BIN_THREADS) void k_bin_scatter(const int* __restri
 
 __global__ void k_set_i32(int* p, int v) { *p = v; }
 
-// The multi-job queue with wave pools: each wave takes a run of 64 *
-// POOL_RAYS consecutive slots and refills its lanes (pool_trace); a lane
-// loads its slot's scene with its ray.
-__global__ __launch_bounds__(256) void k_trace_jobs_pool(const MtSceneRef* __restrict__ refs,
-                                                         const int* __restrict__ tag, int shift, TraceArgs A)
-{
-    int count = *A.d_count;
-    count = count < A.capacity ? count : A.capacity;
-    const int next = (int)(blockIdx.x * 4 + (threadIdx.x >> 6)) * (64 * POOL_RAYS);
-    const int end = count < next + 64 * POOL_RAYS ? count : next + 64 * POOL_RAYS;
-    if (next >= end) return;
-    pool_trace<false>(
-        nullptr, nullptr, 0, next, end,
-        [&](int id, RayT& r, const float4*& pn, const float4*& pt, int& root) {
-            const MtSceneRef R = refs[tag[2 * id] >> shift];
-            pn = R.pn;
-            pt = R.pt;
-            root = R.root;
-            ray_init(r, A.o_tmin[id], A.d_tmax[id]);
-        },
-        [&](bool fin, int id, const RayT& r, const TravState& S) {
-            if (fin) store_result<false, false>(A, id, r, S);
-        });
-}
-
 template <bool ANY>
 int32_t launch_trace(mt_context* ctx, const mt_scene* sc, const float* o_tmin,
                      const float* d_tmax, const int32_t* d_count, int32_t capacity,
@@ -473,7 +374,6 @@ int32_t launch_trace(mt_context* ctx, const mt_scene* sc, const float* o_tmin,
     if (seg.counts) {
         MT_ARG_CHECK(seg.seg_cap % 256 == 0, "trace: segment capacity %d not a multiple of 256", seg.seg_cap);
         capacity = seg.nseg * seg.seg_cap;
-        if (mode == MT_TRACE_PACKED_REFILL) mode = MT_TRACE_PACKED_STACK; // the refill kernel reads *d_count
     }
     if (capacity == 0) return MT_OK;
     TraceArgs A{};
@@ -485,6 +385,7 @@ int32_t launch_trace(mt_context* ctx, const mt_scene* sc, const float* o_tmin,
     A.pn = sc->pnodes;
     A.pt = sc->ptris;
     A.root = sc->root_ref;
+    A.plain = sc->plain;
     A.o_tmin = reinterpret_cast<const float4*>(o_tmin);
     A.d_tmax = reinterpret_cast<const float4*>(d_tmax);
     A.d_count = d_count;
@@ -495,20 +396,21 @@ int32_t launch_trace(mt_context* ctx, const mt_scene* sc, const float* o_tmin,
     A.stats = stats;
     dim3 grid(mt_blocks(capacity, 256)), block(256);
     hipStream_t s = ctx->stream;
-    // Default: one ray per lane with the short stack (8 waves/SIMD).  Refill
-    // wins only on long incoherent batches (16M random any-hit rays through a
-    // 4M-triangle soup: 18.3 vs 21.3 ms); on a path tracer's bounce batches it
-    // loses (1080p x 16 spp render: 25.8 vs 23.5 ms), so it is opt-in.
-    // On the render's segmented bounce queues (secondary rays, incoherent)
-    // the wave pool wins (1080p x 16 spp guided render: bounce-1 closest
-    // hit 2.80 -> 2.21 ms); on coherent batches its desynchronised lanes
-    // fetch more distinct nodes per load and it loses (camera rays 1.40 ->
-    // 1.90 ms), so plain queues keep one ray per lane.
-    if (mode == MT_TRACE_PACKED) mode = seg.counts ? MT_TRACE_PACKED_POOL : MT_TRACE_PACKED_STACK;
-    if ((mode == MT_TRACE_PACKED_SORTED || mode == MT_TRACE_PACKED_POOL || mode == MT_TRACE_PACKED_BINNED) && stats)
-        mode = MT_TRACE_PACKED_STACK; // counting: per-ray order only
-    if (mode == MT_TRACE_PACKED_BINNED && seg.counts) mode = MT_TRACE_PACKED_POOL; // the render's bounce queues
-    if (mode == MT_TRACE_PACKED_BINNED) {
+    if (stats) { // counting: one ray per lane
+        if (mode == MT_TRACE_REFERENCE) k_trace<ANY, true, 1><<<grid, block, 0, s>>>(A);
+        else if (mode == MT_TRACE_PACKED_NO_STACK) k_trace<ANY, true, 2><<<grid, block, 0, s>>>(A);
+        else k_trace<ANY, true, 0><<<grid, block, 0, s>>>(A);
+        MT_LAUNCH_CHECK();
+        return MT_OK;
+    }
+    if (mode == MT_TRACE_REFERENCE || mode == MT_TRACE_PACKED_NO_STACK || mode == MT_TRACE_PACKED_SORTED) {
+        if (mode == MT_TRACE_REFERENCE) k_trace<ANY, false, 1><<<grid, block, 0, s>>>(A);
+        else if (mode == MT_TRACE_PACKED_NO_STACK) k_trace<ANY, false, 2><<<grid, block, 0, s>>>(A);
+        else k_trace_sorted<ANY><<<grid, block, 0, s>>>(A);
+        MT_LAUNCH_CHECK();
+        return MT_OK;
+    }
+    if (mode == MT_TRACE_PACKED_BINNED && !seg.counts) { // (the render's bounce queues trace unsorted)
         // workspace: keys, tile x bin matrix and its scan, the order
         int64_t tile = ((int64_t)capacity + BIN_TILES_TARGET - 1) / BIN_TILES_TARGET;
         tile = tile < BIN_TILE_MIN ? BIN_TILE_MIN : (tile + 1023) & ~(int64_t)1023;
@@ -538,44 +440,29 @@ int32_t launch_trace(mt_context* ctx, const mt_scene* sc, const float* o_tmin,
                                                       (int)tile, order);
         MT_LAUNCH_CHECK();
         A.order = order;
-        // wave pools over the sorted order (64M random rays through 4M
-        // triangles, closest / any hit: 51.0 / 35.7 ms; persistent refill
-        // waves over the same order 63.9 / 39.0 ms): each wave's run is 256
-        // neighbouring rays, whose lanes the pool keeps on nodes
-        mode = MT_TRACE_PACKED_POOL;
     }
-    if (mode == MT_TRACE_PACKED_POOL) {
-        // sorted (binned) batches take runs of 8 rays per lane (64M random
-        // rays, closest / any hit: 49.9 / 34.8 ms against 51.0 / 35.8 with
-        // 4) and a deeper short stack; the render's bounce queues keep 4
-        // rays and 8 entries (8 rays cost its job 1%, 12 entries 0.7%)
-        const int rays = A.order ? BINNED_POOL_RAYS : POOL_RAYS;
-        const int64_t per_group = 256 * (int64_t)rays;
-        const int64_t groups = seg.counts ? (int64_t)seg.nseg * ((seg.seg_cap + per_group - 1) / per_group)
-                                          : (capacity + per_group - 1) / per_group;
-        if (A.order)
-            k_trace_pool<ANY, BINNED_POOL_RAYS, SHORT_STACK_DEEP><<<dim3((unsigned)groups), block, 0, s>>>(A);
-        else k_trace_pool<ANY, POOL_RAYS><<<dim3((unsigned)groups), block, 0, s>>>(A);
-    } else if (mode == MT_TRACE_PACKED_SORTED) {
-        k_trace_sorted<ANY><<<grid, block, 0, s>>>(A);
-    } else if (mode == MT_TRACE_PACKED_REFILL) {
-        void* scr = nullptr;
-        int32_t rc = mt_ctx_scratch(ctx, 256, &scr);
-        if (rc) return rc;
-        // words 0-2: scan look-back ticket, error flag and epoch
-        A.ctr = reinterpret_cast<unsigned*>(scr) + 4;
-        auto kern = stats ? k_trace_refill<ANY, true> : k_trace_refill<ANY, false>;
-        int blocks = mt_persistent_blocks(ctx, kern, 256, capacity);
-        kern<<<blocks, block, 0, s>>>(A);
-    } else if (stats) {
-        if (mode == MT_TRACE_PACKED_STACK) k_trace<ANY, true, 0><<<grid, block, 0, s>>>(A);
-        else if (mode == MT_TRACE_REFERENCE) k_trace<ANY, true, 1><<<grid, block, 0, s>>>(A);
-        else k_trace<ANY, true, 2><<<grid, block, 0, s>>>(A);
-    } else {
-        if (mode == MT_TRACE_PACKED_STACK) k_trace<ANY, false, 0><<<grid, block, 0, s>>>(A);
-        else if (mode == MT_TRACE_REFERENCE) k_trace<ANY, false, 1><<<grid, block, 0, s>>>(A);
-        else k_trace<ANY, false, 2><<<grid, block, 0, s>>>(A);
+    // Form of the walk (WaveForm): a plain queue in the default mode is taken to
+    // be coherent (1.04M camera rays in a room of 20K triangles, closest hit +
+    // shadow ray + any hit: direct 0.96 ms, staged 1.09; start 1.33); the bounce
+    // queues, and the modes for incoherent batches, are staged (16M random rays
+    // through 4M triangles, unsorted, closest + any: staged with the deep stack
+    // 28.0 ms, direct 30.7; start 29.4; sorted 15.9, with 9 rows 16.9, start 22.7).
+    const bool wide = scene_wide(sc);
+    auto kern = wide ? k_trace_wave<ANY, true, WT_DIRECT> : k_trace_wave<ANY, false, WT_DIRECT>;
+    int slots = WaveLds<WT_DIRECT>::SLOTS;
+    if (A.order) {
+        kern = wide ? k_trace_wave<ANY, true, WT_STAGED_DEEP> : k_trace_wave<ANY, false, WT_STAGED_DEEP>;
+    } else if (seg.counts) {
+        kern = wide ? k_trace_wave<ANY, true, WT_STAGED> : k_trace_wave<ANY, false, WT_STAGED>;
+        slots = WaveLds<WT_STAGED>::SLOTS;
+    } else if (mode == MT_TRACE_PACKED_POOL || mode == MT_TRACE_PACKED_REFILL) {
+        kern = wide ? k_trace_wave<ANY, true, WT_STAGED_DEEP> : k_trace_wave<ANY, false, WT_STAGED_DEEP>;
+        slots = WaveLds<WT_STAGED_DEEP>::SLOTS;
     }
+    A.run = A.order ? WT_BINNED_RUN : wave_run(capacity, slots);
+    const int64_t groups = seg.counts ? (int64_t)seg.nseg * wave_seg_groups(seg.seg_cap, seg.nseg, slots)
+                                      : (capacity + 4 * (int64_t)A.run - 1) / (4 * (int64_t)A.run);
+    kern<<<dim3((unsigned)groups), block, 0, s>>>(A);
     MT_LAUNCH_CHECK();
     return MT_OK;
 }
@@ -592,8 +479,11 @@ __global__ void k_leaf_flags(const int* __restrict__ nodes, int n, int* __restri
 // Range checks of every index the traversal follows.  err bit 1: node link
 // out of range; 2: face vertex out of range; 4: leaf primitive out of range;
 // 8: bound index != own index (the reference's invariant, CNormalBVH.java:88).
-__global__ void k_validate(const int* __restrict__ nodes, int nn, const int* __restrict__ faces,
-                           int ntris, int npoints, int* err)
+// 256 is no error: some box is inverted, not finite or beyond 1e30
+// (mt_scene::plain is then 0).
+constexpr int BOXES_NOT_PLAIN = 256;
+__global__ void k_validate(const int* __restrict__ nodes, const float* __restrict__ bounds, int nn,
+                           const int* __restrict__ faces, int ntris, int npoints, int* err)
 {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
     int e = 0;
@@ -606,6 +496,9 @@ __global__ void k_validate(const int* __restrict__ nodes, int nn, const int* __r
             if (n[2] <= 0 || n[2] >= nn || n[3] <= 0 || n[3] >= nn) e |= 1;
         }
         if (n[1] < 0 || n[1] >= nn || n[4] < 0 || n[4] >= nn) e |= 1;
+        const float* b = bounds + 8 * (size_t)i;
+        for (int a = 0; a < 3; a++)
+            if (!(b[a] <= b[4 + a] && b[a] >= -1e30f && b[4 + a] <= 1e30f)) e |= BOXES_NOT_PLAIN;
     }
     if (i < ntris) {
         const int* F = faces + 10 * i;
@@ -656,9 +549,7 @@ __global__ void k_pack(const int* __restrict__ nodes, const float* __restrict__ 
         const float* lb = bounds + 8 * nodes[7 * n[2]];
         const float* rb = bounds + 8 * nodes[7 * n[3]];
         float4* N = pn + 4 * (size_t)(i - leaf_rank[i]);
-        N[0] = make_float4(lb[0], lb[1], lb[2], lb[4]);
-        N[1] = make_float4(lb[5], lb[6], rb[0], rb[1]);
-        N[2] = make_float4(rb[2], rb[4], rb[5], rb[6]);
+        for (int a = 0; a < 3; a++) N[a] = make_float4(lb[a], rb[a], lb[4 + a], rb[4 + a]);
         int parent = n[4];
         int4 d = make_int4(ref(n[2]), ref(n[3]), parent - leaf_rank[parent], ref(n[1]));
         N[3] = *reinterpret_cast<float4*>(&d);
@@ -799,42 +690,34 @@ __global__ __launch_bounds__(256) void k_shade(const float4* __restrict__ points
 // distance into the ray's tMax (intersectMesh, NormalBVH.cl:42); a miss,
 // and every slot in [*count, capacity), writes hit = 0 and mat = -1 and
 // leaves the other fields as they were.
-template <int LAYOUT>
-__global__ __launch_bounds__(256) void k_intersect_records(TraceArgs A, const float4* __restrict__ normals,
-                                                           const float2* __restrict__ uvs, float4* rays,
-                                                           float4* isects)
+__device__ __forceinline__ void record_ray(const float4* R, RayT& r)
 {
-    const int id = blockIdx.x * blockDim.x + threadIdx.x;
-    if (id >= A.capacity) return;
+    const float4 o4 = R[0], d4 = R[1], inv4 = R[2], sg = R[3], ex = R[4];
+    r.o = mk3(o4.x, o4.y, o4.z);
+    r.d = mk3(d4.x, d4.y, d4.z);
+    r.inv = mk3(inv4.x, inv4.y, inv4.z);
+    r.sx = __float_as_int(sg.x) != 0;
+    r.sy = __float_as_int(sg.y) != 0;
+    r.sz = __float_as_int(sg.z) != 0;
+    r.tmin = ex.z;
+    r.tmax = ex.w;
+}
+
+// Slot id's outcome: primitive `child` at distance t (child < 0: a miss).
+__device__ __forceinline__ void record_result(const TraceArgs& A, const float4* __restrict__ normals,
+                                              const float2* __restrict__ uvs, float4* rays, float4* isects, int id,
+                                              int child, float t)
+{
     int* iw = reinterpret_cast<int*>(isects + 6 * (size_t)id);
-    float4* R = rays + 5 * (size_t)id;
-    int child = -1;
-    int h = 0;
-    RayT r;
-    float4 d4 = make_float4(0, 0, 0, 0);
-    if (entry_live(A, id)) {
-        const float4 o4 = R[0], inv4 = R[2], sg = R[3], ex = R[4];
-        d4 = R[1];
-        r.o = mk3(o4.x, o4.y, o4.z);
-        r.d = mk3(d4.x, d4.y, d4.z);
-        r.inv = mk3(inv4.x, inv4.y, inv4.z);
-        r.sx = __float_as_int(sg.x) != 0;
-        r.sy = __float_as_int(sg.y) != 0;
-        r.sz = __float_as_int(sg.z) != 0;
-        r.tmin = ex.z;
-        r.tmax = ex.w;
-        int st[3];
-        h = LAYOUT == 0   ? trace_packed<false, false, true>(A.pn, A.pt, A.root, r, child, st)
-            : LAYOUT == 2 ? trace_packed<false, false, false>(A.pn, A.pt, A.root, r, child, st)
-                          : trace_reference<false, false>(A.nodes, A.bounds, A.faces, A.points, r, child, st);
-    }
-    if (!h) {
+    if (child < 0) {
         iw[18] = -1; // mat
         iw[20] = 0;  // hit = MISS_MARKER
         return;
     }
-    reinterpret_cast<float*>(R)[19] = r.tmax;
-    const HitShading H = hit_shading(A.points, normals, uvs, A.faces, r.o, r.d, child, r.tmax);
+    float4* R = rays + 5 * (size_t)id;
+    const float4 o4 = R[0], d4 = R[1];
+    reinterpret_cast<float*>(R)[19] = t;
+    const HitShading H = hit_shading(A.points, normals, uvs, A.faces, xyz(o4), xyz(d4), child, t);
     float4* I = isects + 6 * (size_t)id;
     I[0] = H.p;
     I[1] = H.n;
@@ -844,30 +727,86 @@ __global__ __launch_bounds__(256) void k_intersect_records(TraceArgs A, const fl
     iw[20] = 1; // hit = HIT_MARKER
 }
 
+// The packed layout: each wave traces a run of slots (wave_trace); LAYOUT 1
+// and 2 below trace one slot per lane over the reference arrays or without a
+// stack.
+template <bool WIDE>
+__global__ __launch_bounds__(256, WaveLds<WT_DIRECT>::WAVES) void k_intersect_records_wave(TraceArgs A, const float4* __restrict__ normals,
+                                                                           const float2* __restrict__ uvs,
+                                                                           float4* rays, float4* isects)
+{
+    __shared__ WaveLds<WT_DIRECT> s_w[4];
+    int count = *A.d_count;
+    count = count < A.capacity ? count : A.capacity;
+    count = count > 0 ? count : 0;
+    const int64_t first = ((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * A.run;
+    if (first >= A.capacity) return;
+    const int next = (int)first;
+    const int stop = A.capacity - next < A.run ? A.capacity : next + A.run;
+    // slots past *d_count are misses
+    for (int id = (next > count ? next : count) + (int)__lane_id(); id < stop; id += 64)
+        record_result(A, normals, uvs, rays, isects, id, -1, 0.0f);
+    const int end = count < stop ? count : stop;
+    if (next >= end) return;
+    wave_trace<false, WIDE, WT_REFILL>(
+        s_w, MtSceneRef{A.pn, A.pt, A.root, A.plain}, next, end,
+        [&](int id, RayT& r, MtSceneRef&) { record_ray(rays + 5 * (size_t)id, r); },
+        [&](bool fin, int id, float t, int child, const MtSceneRef&) {
+            if (fin) record_result(A, normals, uvs, rays, isects, id, leaf_prim(A.pt, child), t);
+        });
+}
+
+template <int LAYOUT>
+__global__ __launch_bounds__(256) void k_intersect_records(TraceArgs A, const float4* __restrict__ normals,
+                                                           const float2* __restrict__ uvs, float4* rays,
+                                                           float4* isects)
+{
+    const int id = blockIdx.x * blockDim.x + threadIdx.x;
+    if (id >= A.capacity) return;
+    int child = -1;
+    int h = 0;
+    RayT r;
+    if (entry_live(A, id)) {
+        record_ray(rays + 5 * (size_t)id, r);
+        int st[3];
+        h = LAYOUT == 2 ? trace_packed<false, false, false>(A.pn, A.pt, A.root, r, child, st)
+                        : trace_reference<false, false>(A.nodes, A.bounds, A.faces, A.points, r, child, st);
+    }
+    record_result(A, normals, uvs, rays, isects, id, h ? child : -1, r.tmax);
+}
+
 // intersectOcclusion (NormalBVH.cl:319-348) over Ray records: intersectMesh
 // with bailout, i.e. any hit in the reference's visiting order, the ray left
 // unchanged; hits[id] written for id < *count only.
+template <bool WIDE>
+__global__ __launch_bounds__(256, WaveLds<WT_DIRECT>::WAVES) void k_occlusion_records_wave(TraceArgs A, const float4* __restrict__ rays, int* hits)
+{
+    __shared__ WaveLds<WT_DIRECT> s_w[4];
+    int count = *A.d_count;
+    count = count < A.capacity ? count : A.capacity;
+    const int64_t first = ((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * A.run;
+    if (first >= count) return;
+    const int next = (int)first;
+    const int end = count - next < A.run ? count : next + A.run;
+    wave_trace<true, WIDE, WT_REFILL>(
+        s_w, MtSceneRef{A.pn, A.pt, A.root, A.plain}, next, end,
+        [&](int id, RayT& r, MtSceneRef&) { record_ray(rays + 5 * (size_t)id, r); },
+        [&](bool fin, int id, float, int child, const MtSceneRef&) {
+            if (fin) hits[id] = child != WT_NONE;
+        });
+}
+
 template <int LAYOUT>
 __global__ __launch_bounds__(256) void k_occlusion_records(TraceArgs A, const float4* __restrict__ rays, int* hits)
 {
     const int id = blockIdx.x * blockDim.x + threadIdx.x;
     if (!entry_live(A, id)) return;
-    const float4* R = rays + 5 * (size_t)id;
-    const float4 o4 = R[0], d4 = R[1], inv4 = R[2], sg = R[3], ex = R[4];
     RayT r;
-    r.o = mk3(o4.x, o4.y, o4.z);
-    r.d = mk3(d4.x, d4.y, d4.z);
-    r.inv = mk3(inv4.x, inv4.y, inv4.z);
-    r.sx = __float_as_int(sg.x) != 0;
-    r.sy = __float_as_int(sg.y) != 0;
-    r.sz = __float_as_int(sg.z) != 0;
-    r.tmin = ex.z;
-    r.tmax = ex.w;
+    record_ray(rays + 5 * (size_t)id, r);
     int st[3];
     int child = -1;
-    hits[id] = LAYOUT == 0   ? trace_packed<true, false, true>(A.pn, A.pt, A.root, r, child, st)
-               : LAYOUT == 2 ? trace_packed<true, false, false>(A.pn, A.pt, A.root, r, child, st)
-                             : trace_reference<true, false>(A.nodes, A.bounds, A.faces, A.points, r, child, st);
+    hits[id] = LAYOUT == 2 ? trace_packed<true, false, false>(A.pn, A.pt, A.root, r, child, st)
+                           : trace_reference<true, false>(A.nodes, A.bounds, A.faces, A.points, r, child, st);
 }
 
 __global__ __launch_bounds__(256) void k_shadow_rays(const float4* __restrict__ o_tmin,
@@ -939,7 +878,7 @@ extern "C" int32_t mt_scene_create(mt_context* ctx, const mt_scene_desc* desc, m
     hipStream_t s = ctx->stream;
     int32_t rc = mt_buf_fill_i32(ctx, err, 0, 2);
     if (rc) return fail(rc);
-    k_validate<<<mt_blocks(nn, 256), 256, 0, s>>>(desc->nodes, nn, desc->faces, desc->num_tris,
+    k_validate<<<mt_blocks(nn, 256), 256, 0, s>>>(desc->nodes, desc->bounds, nn, desc->faces, desc->num_tris,
                                                   desc->num_points, err);
     int herr = 0;
     if (hipGetLastError() != hipSuccess ||
@@ -948,7 +887,8 @@ extern "C" int32_t mt_scene_create(mt_context* ctx, const mt_scene_desc* desc, m
         mt_set_error("mt_scene_create: validation launch failed");
         return fail(MT_ERR_HIP);
     }
-    if (herr) {
+    sc->plain = herr & BOXES_NOT_PLAIN ? 0 : 1;
+    if (herr & ~BOXES_NOT_PLAIN) {
         mt_set_error("mt_scene_create: invalid scene arrays (error mask 0x%x: 1 node link, "
                      "2 face vertex, 4 leaf primitive, 8 bound index)", herr);
         return fail(MT_ERR_ARG);
@@ -960,7 +900,7 @@ extern "C" int32_t mt_scene_create(mt_context* ctx, const mt_scene_desc* desc, m
         mt_set_error("mt_scene_create: depth check launch failed");
         return fail(MT_ERR_HIP);
     }
-    if (herr) {
+    if (herr & ~BOXES_NOT_PLAIN) {
         mt_set_error("mt_scene_create: BVH deeper than 128 levels or parent links broken");
         return fail(MT_ERR_DEPTH);
     }
@@ -1017,8 +957,8 @@ extern "C" int32_t mt_trace_autotune(mt_context* ctx, const mt_scene* scene, con
     MT_ARG_CHECK(ctx && scene && best_mode && best_ms, "mt_trace_autotune: NULL argument");
     MT_ARG_CHECK(reps >= 1 && reps <= 100, "mt_trace_autotune: reps %d not in [1,100]", reps);
     MT_ARG_CHECK(any ? occluded != nullptr : (prim && t), "mt_trace_autotune: NULL outputs");
-    const int32_t modes[4] = {MT_TRACE_PACKED_STACK, MT_TRACE_PACKED_REFILL, MT_TRACE_PACKED_POOL,
-                              MT_TRACE_PACKED_BINNED};
+    // (MT_TRACE_PACKED_POOL is the same kernel as _REFILL)
+    const int32_t modes[3] = {MT_TRACE_PACKED_STACK, MT_TRACE_PACKED_REFILL, MT_TRACE_PACKED_BINNED};
     hipEvent_t e0 = nullptr, e1 = nullptr;
     MT_HIP_CHECK(hipEventCreate(&e0));
     if (hipEventCreate(&e1) != hipSuccess) {
@@ -1084,7 +1024,7 @@ int32_t mt_trace_any_seg(mt_context* ctx, const mt_scene* scene, const float4* o
 
 int32_t mt_trace_jobs(mt_context* ctx, const MtSceneRef* refs, const int32_t* tag, int32_t shift,
                       const float4* o_tmin, const float4* d_tmax, const int32_t* d_count, int32_t capacity,
-                      int32_t* prim, float* t, int32_t mode, const int32_t* d_split)
+                      int32_t* prim, float* t)
 {
     if (capacity == 0) return MT_OK;
     TraceArgs A{};
@@ -1094,20 +1034,8 @@ int32_t mt_trace_jobs(mt_context* ctx, const MtSceneRef* refs, const int32_t* ta
     A.capacity = capacity;
     A.prim = prim;
     A.tout = t;
-    if (mode == MT_BATCH_TRACE_SPLIT) {
-        MT_ARG_CHECK(d_split, "mt_trace_jobs: the split mode needs the survivors' count");
-        // survivors (incoherent secondary rays) with wave pools ...
-        TraceArgs P = A;
-        P.d_count = d_split;
-        k_trace_jobs_pool<<<mt_blocks(capacity, 256 * POOL_RAYS), 256, 0, ctx->stream>>>(refs, tag, shift, P);
-        MT_LAUNCH_CHECK();
-        // ... and the new camera rays (coherent) one per lane
-        k_trace_jobs<<<mt_blocks(capacity, 256), 256, 0, ctx->stream>>>(refs, tag, shift, A, d_split);
-    } else if (mode == MT_TRACE_PACKED_POOL) {
-        k_trace_jobs_pool<<<mt_blocks(capacity, 256 * POOL_RAYS), 256, 0, ctx->stream>>>(refs, tag, shift, A);
-    } else {
-        k_trace_jobs<<<mt_blocks(capacity, 256), 256, 0, ctx->stream>>>(refs, tag, shift, A, nullptr);
-    }
+    A.run = wave_run(capacity, WaveLds<WT_STAGED>::SLOTS);
+    k_trace_jobs<<<mt_blocks(capacity, 4 * A.run), 256, 0, ctx->stream>>>(refs, tag, shift, A);
     MT_LAUNCH_CHECK();
     return MT_OK;
 }
@@ -1149,6 +1077,7 @@ extern "C" int32_t mt_intersect_primitives(mt_context* ctx, const mt_scene* sc, 
     A.pn = sc->pnodes;
     A.pt = sc->ptris;
     A.root = sc->root_ref;
+    A.plain = sc->plain;
     A.d_count = d_count;
     A.capacity = capacity;
     const float4* nrm = reinterpret_cast<const float4*>(sc->desc.normals);
@@ -1157,10 +1086,13 @@ extern "C" int32_t mt_intersect_primitives(mt_context* ctx, const mt_scene* sc, 
     float4* I = reinterpret_cast<float4*>(isects);
     dim3 grid(mt_blocks(capacity, 256)), block(256);
     hipStream_t s = ctx->stream;
-    // every packed mode gives the same bits; this writer runs one ray per lane
+    // every other packed mode gives the same bits: one kernel
+    A.run = wave_run(capacity, WaveLds<WT_DIRECT>::SLOTS);
+    const int waves = mt_blocks(capacity, 4 * A.run);
     if (mode == MT_TRACE_REFERENCE) k_intersect_records<1><<<grid, block, 0, s>>>(A, nrm, uvs, R, I);
     else if (mode == MT_TRACE_PACKED_NO_STACK) k_intersect_records<2><<<grid, block, 0, s>>>(A, nrm, uvs, R, I);
-    else k_intersect_records<0><<<grid, block, 0, s>>>(A, nrm, uvs, R, I);
+    else if (scene_wide(sc)) k_intersect_records_wave<true><<<waves, block, 0, s>>>(A, nrm, uvs, R, I);
+    else k_intersect_records_wave<false><<<waves, block, 0, s>>>(A, nrm, uvs, R, I);
     MT_LAUNCH_CHECK();
     return MT_OK;
 }
@@ -1182,14 +1114,17 @@ extern "C" int32_t mt_intersect_occlusion(mt_context* ctx, const mt_scene* sc, c
     A.pn = sc->pnodes;
     A.pt = sc->ptris;
     A.root = sc->root_ref;
+    A.plain = sc->plain;
     A.d_count = d_count;
     A.capacity = capacity;
     const float4* R = reinterpret_cast<const float4*>(rays);
     dim3 grid(mt_blocks(capacity, 256)), block(256);
     hipStream_t s = ctx->stream;
+    A.run = wave_run(capacity, WaveLds<WT_DIRECT>::SLOTS);
     if (mode == MT_TRACE_REFERENCE) k_occlusion_records<1><<<grid, block, 0, s>>>(A, R, hits);
     else if (mode == MT_TRACE_PACKED_NO_STACK) k_occlusion_records<2><<<grid, block, 0, s>>>(A, R, hits);
-    else k_occlusion_records<0><<<grid, block, 0, s>>>(A, R, hits);
+    else if (scene_wide(sc)) k_occlusion_records_wave<true><<<mt_blocks(capacity, 4 * A.run), block, 0, s>>>(A, R, hits);
+    else k_occlusion_records_wave<false><<<mt_blocks(capacity, 4 * A.run), block, 0, s>>>(A, R, hits);
     MT_LAUNCH_CHECK();
     return MT_OK;
 }

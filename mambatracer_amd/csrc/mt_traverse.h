@@ -59,7 +59,9 @@ __device__ __forceinline__ float tri_hit(const RayT& r, v3 p1, v3 e1, v3 e2)
 {
     const v3 h = cross3(r.d, e2);
     const float a = dot3(e1, h);
-    const bool parallel = ((double)a > -0.0000001) & ((double)a < 0.0000001); // double compare, :13
+    // :13 compares a with the double 0.0000001; 0x33d6bf94 (9.9999994e-8) is
+    // the largest float below it, so in floats the test is |a| <= that
+    const bool parallel = fabsf(a) <= __int_as_float(0x33d6bf94);
     const float f = 1.0f / a;
     const v3 s = sub3(r.o, p1);
     const float b1 = f * dot3(s, h);
@@ -112,8 +114,7 @@ struct BitStack {
 // record's last word pair, a leaf triangle's spare words), so no links are
 // carried in registers while descending.  Depth N is a trade: each push
 // and pop moves N registers, and a deeper stack saves parent walks on deep
-// trees.  MT_SHORT_STACK (8) serves the render's 1M-triangle scene; the wave
-// pools over sorted batches of deep trees use SHORT_STACK_DEEP.
+// trees.
 #ifndef MT_SHORT_STACK
 #define MT_SHORT_STACK 8
 #endif
@@ -211,7 +212,6 @@ __device__ __forceinline__ int trace_reference(const int* __restrict__ nodes,
 // cur < 0: leaf ~rank.  parent/sib track the current node's links, which the
 // reference reads from the node records (leaves are not records here).
 // -------------------------------------------------------------------------
-// Resumable traversal state of one ray (packed layout).
 // Parent and sibling references of node `cur`: an interior record's last
 // word pair, or the spare words of a leaf's triangle record.
 __device__ __forceinline__ int2 node_links(const float4* __restrict__ pn, const float4* __restrict__ pt, int cur)
@@ -240,140 +240,9 @@ __device__ __forceinline__ bool parent_walk(const float4* __restrict__ pn, const
     return true;
 }
 
-// Resumable traversal state of one ray (packed layout), short stack of N.
-template <int N>
-struct TravStateN {
-    int cur;
-    BitStack bs;
-    ShortStackN<N> ss;
-    int hit, child;
-    int st[3];
-    __device__ __forceinline__ void init(int root)
-    {
-        cur = root;
-        bs.lo = 0;
-        bs.hi = 0;
-        ss.n = 0;
-        hit = 0;
-        child = -1;
-        st[0] = st[1] = st[2] = 0;
-    }
-};
-using TravState = TravStateN<MT_SHORT_STACK>;
-
-// One outer iteration of the packed traversal: descend to a leaf (or a node
-// whose children both miss), test the leaf, move to the next pending subtree.
-// Returns true when the ray is finished.  The sequence of nodes visited over
-// all iterations is exactly the reference's (see trace_packed below).
-template <bool ANY, bool STATS, bool SHORT_STACK>
-__device__ __forceinline__ bool trace_packed_step(const float4* __restrict__ pn, const float4* __restrict__ pt,
-                                                  RayT& r, TravState& S)
-{
-    while (S.cur >= 0) {
-        const float4* N = pn + 4 * (size_t)S.cur;
-        float4 a = N[0], b = N[1], c = N[2];
-        int4 d = *reinterpret_cast<const int4*>(N + 3);
-        float lt, rt;
-        bool lh = box_hit(r, a.x, a.y, a.z, a.w, b.x, b.y, lt);
-        bool rh = box_hit(r, b.z, b.w, c.x, c.y, c.z, c.w, rt);
-        if (STATS) S.st[0]++;
-        if (!lh && !rh) break;
-        S.bs.push0();
-        int nxt;
-        if (lh && rh) {
-            bool right_first = rt < lt;
-            nxt = right_first ? d.y : d.x;
-            if (SHORT_STACK) S.ss.push(right_first ? d.x : d.y);
-            S.bs.lo |= 1;
-        } else {
-            nxt = lh ? d.x : d.y;
-        }
-        S.cur = nxt;
-    }
-    if (S.cur < 0) {
-        if (STATS) S.st[1]++;
-        const float4* T = pt + 3 * (size_t)(~S.cur);
-        float4 t0 = T[0], t1 = T[1], t2 = T[2];
-        float t = tri_hit(r, mk3(t0.x, t0.y, t0.z), mk3(t0.w, t1.x, t1.y), mk3(t1.z, t1.w, t2.x));
-        if ((r.tmin < t) && (t < r.tmax)) {
-            S.hit = 1;
-            if (ANY) return true;
-            r.tmax = t;
-            S.child = __float_as_int(t2.y);
-        }
-    }
-    if (S.bs.empty()) return true;
-    if (SHORT_STACK && S.ss.n > 0) {
-        int z = S.bs.ctz();
-        if (STATS) S.st[2] += z;
-        S.bs.shr(z);
-        S.bs.lo ^= 1;
-        S.cur = S.ss.pop();
-        return false;
-    }
-    return !parent_walk<STATS>(pn, pt, S.cur, S.bs, S.st);
-}
-
 __device__ __forceinline__ uint32_t lane_rank(uint64_t mask)
 { // set bits of `mask` below this lane (v_mbcnt_lo/hi)
     return __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
-}
-
-// One node of the packed traversal per call: an interior node's box pair
-// (descending to the chosen child, or moving to the next pending subtree
-// when both miss) or a leaf's triangle (then moving on).  Returns true when
-// the ray is finished.  Successive calls visit exactly the nodes of
-// trace_packed_step in the same order; a wave that calls this in a loop
-// keeps every lane on a node of its own ray each iteration instead of
-// holding the lanes that reached a leaf until the whole wave has.
-template <bool ANY, bool STATS, int DEPTH>
-__device__ __forceinline__ bool trace_packed_node(const float4* __restrict__ pn, const float4* __restrict__ pt,
-                                                  RayT& r, TravStateN<DEPTH>& S)
-{
-    if (S.cur >= 0) {
-        const float4* N = pn + 4 * (size_t)S.cur;
-        float4 a = N[0], b = N[1], c = N[2];
-        int4 d = *reinterpret_cast<const int4*>(N + 3);
-        float lt, rt;
-        bool lh = box_hit(r, a.x, a.y, a.z, a.w, b.x, b.y, lt);
-        bool rh = box_hit(r, b.z, b.w, c.x, c.y, c.z, c.w, rt);
-        if (STATS) S.st[0]++;
-        if (lh || rh) {
-            S.bs.push0();
-            int nxt;
-            if (lh && rh) {
-                bool right_first = rt < lt;
-                nxt = right_first ? d.y : d.x;
-                S.ss.push(right_first ? d.x : d.y);
-                S.bs.lo |= 1;
-            } else {
-                nxt = lh ? d.x : d.y;
-            }
-            S.cur = nxt;
-            return false;
-        }
-    } else {
-        if (STATS) S.st[1]++;
-        const float4* T = pt + 3 * (size_t)(~S.cur);
-        float4 t0 = T[0], t1 = T[1], t2 = T[2];
-        float t = tri_hit(r, mk3(t0.x, t0.y, t0.z), mk3(t0.w, t1.x, t1.y), mk3(t1.z, t1.w, t2.x));
-        if ((r.tmin < t) && (t < r.tmax)) {
-            S.hit = 1;
-            if (ANY) return true;
-            r.tmax = t;
-            S.child = __float_as_int(t2.y);
-        }
-    }
-    if (S.bs.empty()) return true;
-    if (S.ss.n > 0) {
-        int z = S.bs.ctz();
-        if (STATS) S.st[2] += z;
-        S.bs.shr(z);
-        S.bs.lo ^= 1;
-        S.cur = S.ss.pop();
-        return false;
-    }
-    return !parent_walk<STATS>(pn, pt, S.cur, S.bs, S.st);
 }
 
 // Work-groups go to the 8 XCDs in turn (group b on XCD b mod 8), each XCD
@@ -418,82 +287,378 @@ __device__ __forceinline__ unsigned seg_sweep_group()
     return xcd_chunked_group(blockIdx.x, gridDim.x, XCD_RUN);
 }
 
-// Idle lanes a pool waits for before starting new rays.
-constexpr int POOL_REFILL_MIN = 16;
+// ---------------------------------------------------------------------------
+// Wave traversal: one ray per lane of a wave, every ray in the reference's
+// visiting order (the packed layout of trace_packed below).
+//
+// What bounds it on gfx950: vector issue and the vector L1.  Measured rates
+// per wave64 instruction and SIMD: 2.4 cycles for f32 add / mul, moves, integer
+// add and logic; 4.2-4.5 for compares, selects, min / max (also of three),
+// DPP and shift-adds.  The L1 looks one 64-byte piece up per cycle, and four
+// 16-byte loads of a node by lanes that hold different nodes are four pieces
+// per lane.  So:
+//  * a lane's pending subtrees are a plain stack of references in LDS (one
+//    write and one read per step, both unconditional) instead of a register
+//    queue moved on every push and pop and a 128-bit bitstack; entries past
+//    the LDS rows go to scratch memory, which only deep trees reach;
+//  * a step has no branches: lanes without an interior node run along and
+//    keep their state by selects;
+//  * the slab test is max3 / min3 (20 instead of 30 instructions per box)
+//    wherever no NaN can arise, intersectBoundT's chain otherwise (slab);
+//  * leaves wait until a quarter of the wave's rays are at one, or done
+//    (tried: an eighth to a half), so the triangle test runs for many lanes
+//    instead of interrupting the walk for one or two;
+//  * lanes whose ray has ended take the next of the wave's run together.
+// Node records reach the lanes in one of two ways (WaveForm):
+//  * direct: each lane loads its own record (four loads); near and far planes
+//    picked by selects.  8 waves per SIMD.  Best where neighbouring lanes hold the
+//    same node (camera rays, shadow rays) or rays are short.
+//  * staged: the four lanes of a quad load each of their four records
+//    together, 16 bytes per lane, straight into LDS
+//    (global_load_lds_dwordx4), so a record is one L1 piece instead of
+//    four; every lane then reads its near and its far planes from LDS with
+//    addresses that hold its ray's signs, so nothing is selected.  LDS limits it to 6 waves
+//    per SIMD, 5 with a deeper stack.  Best on incoherent rays with long walks.
+// Measured, start of this design (register queue and bitstack, leaf tests
+// mixed into every step) against now: closest hit of 16M random rays sorted by
+// origin through 4M triangles 12.9 -> 8.6 ms (staged; VALU instructions
+// 8.9 -> 3.6 G, active lanes 25 -> 46 of 64, L1 pieces 6.2 -> 2.7 G);
+// 1920x1080 x 16 spp camera rays through 1M triangles 1.34 -> 1.24 ms (direct;
+// staged 1.54), the 16M shadow rays of its first hits 1.65 -> 1.44 ms (direct;
+// staged 1.81); first bounce of 993K rays in a soup of 150K triangles
+// 0.98 -> 0.61 ms (staged; direct 0.65).
+// ---------------------------------------------------------------------------
+constexpr int WT_NONE = (int)0x80000000; // no node (never a leaf reference: ranks stay below 2^30)
+constexpr int WT_SLOT = 1040;            // bytes between a wave's four load slots: 16 past 1024, so
+                                         // that a quad's records lie in different LDS banks
+constexpr int WT_REFILL = 16;            // idle lanes a wave waits for before starting new rays
+constexpr int WT_REFILL_ANY = 32;        // the same for shadow rays, whose end costs more (any of 16 .. 48: within 1%)
+constexpr int WT_REFILL_CAMERA = 64;     // camera rays start and end together; making one costs ~200 instructions
+constexpr int WT_OVF = 128;              // stack entries in scratch memory: trees are at most 128 deep, a pending
+                                         // subtree per level at most
+constexpr int WT_MIN_RUN = 16;           // rays per wave, at least, and
+constexpr int WT_MAX_RUN = 256;          //   at most while that fills the GPU's wave slots
+constexpr int WT_BINNED_RUN = 512;       // rays per wave of a sorted batch: neighbours share nodes
 
-// Wave-pool traversal of the rays of entries [next, end) (wave-uniform): the
-// wave starts one ray per lane, every iteration takes each lane one node
-// further on its ray (trace_packed_node), and once POOL_REFILL_MIN lanes'
-// rays have ended those lanes take the run's next entries in lane order
-// (ballot + mbcnt on a wave-uniform cursor; no atomics), so lanes stay busy
-// until the run is drained: a
-// wave's tail, where its longest rays run while the other lanes idle, comes
-// once per run instead of once per 64 rays.  load(id, r, pn, pt, root)
-// initialises entry id's ray (and may set the lane's scene: every lane
-// starts on the caller's); done(fin, id, r, S) is called after every
-// iteration with the whole wave active, fin set on the lanes whose ray ended
-// in it.  Each ray is traversed in the reference's
-// visiting order; only the lane that computes it changes.
-template <bool ANY, int N = MT_SHORT_STACK, class Load, class Done>
-__device__ __forceinline__ void pool_trace(const float4* __restrict__ pn, const float4* __restrict__ pt, int root,
-                                           int next, int end, Load&& load, Done&& done)
+enum WaveForm { WT_DIRECT, WT_STAGED, WT_STAGED_DEEP };
+
+template <WaveForm F>
+struct WaveLds {
+    static constexpr int ROWS = F == WT_DIRECT ? 12 : F == WT_STAGED ? 9 : 14; // pending subtrees per lane
+    static constexpr int WAVES = F == WT_DIRECT ? 8 : F == WT_STAGED ? 6 : 5;  // per SIMD
+    static constexpr int SLOTS = 1024 * WAVES; // waves that the GPU's 1024 SIMDs hold at once
+    char node[F == WT_DIRECT ? 256 : 4 * WT_SLOT]; // direct: only the row under the stack, which idle lanes read
+    int stack[ROWS + 1][64];                       // row 0: WT_NONE under the bottom
+};
+typedef __attribute__((address_space(3))) char lds_char;
+typedef __attribute__((address_space(3))) int lds_int;
+typedef float vf2 __attribute__((ext_vector_type(2)));
+typedef int vi2 __attribute__((ext_vector_type(2)));
+
+__device__ __forceinline__ vf2 lds_pair(int addr) { return *(__attribute__((address_space(3))) vf2*)addr; }
+__device__ __forceinline__ lds_int& lds_word(int addr) { return *(lds_int*)addr; }
+
+// Lane J's value of each quad, in all four lanes.
+template <int J>
+__device__ __forceinline__ int quad_bcast(int v)
 {
-    bool active = false;
+    return __builtin_amdgcn_mov_dpp(v, J * 0x55, 0xf, 0xf, true);
+}
+
+struct WaveRay {
+    v3 o, d, inv;
+    float tmin, tmax;
+    int cur;        // node to visit: >= 0 interior, < 0 leaf ~rank, WT_NONE
+    int child;      // leaf of the closest hit so far, WT_NONE: none
+    int sp;         // LDS address of the row above the newest pending subtree
+    int nx, ny, nz; // staged: LDS address of the near planes' pair per axis (less 16 per axis);
+    int fx, fy, fz; //   and of the far planes'.  Direct: nx .. nz nonzero where inv < 0
+};
+
+// Whether max3 / min3 give intersectBoundT's result for this ray in a plain
+// scene (mt_scene::plain): no product can be NaN (inv finite and not 0, origin and
+// planes within 1e30) and the sign words say what inv does, so that per axis
+// near <= far.
+__device__ __forceinline__ bool ray_plain(const RayT& r)
+{
+    auto ok = [](float inv, float o, int s) {
+        const float a = fabsf(inv);
+        return a > 0.0f && a < INFINITY && fabsf(o) < 1e30f && (s != 0) == (inv < 0.0f);
+    };
+    return ok(r.inv.x, r.o.x, r.sx) && ok(r.inv.y, r.o.y, r.sy) && ok(r.inv.z, r.o.z, r.sz);
+}
+
+__device__ __forceinline__ void wave_ray_start(WaveRay& R, const RayT& r, int slot, int col, int root)
+{
+    R.o = r.o;
+    R.d = r.d;
+    R.inv = r.inv;
+    R.tmin = r.tmin;
+    R.tmax = r.tmax;
+    R.cur = root;
+    R.child = WT_NONE;
+    // the last ray's last pop left sp at this row, and until the lane takes a
+    // ray again the steps of the other lanes write there
+    lds_word(col) = WT_NONE;
+    R.sp = col + 256;
+    const int sx = r.sx ? 8 : 0, sy = r.sy ? 8 : 0, sz = r.sz ? 8 : 0;
+    R.nx = slot + sx;
+    R.ny = slot + sy;
+    R.nz = slot + sz;
+    R.fx = slot + 8 - sx;
+    R.fy = slot + 8 - sy;
+    R.fz = slot + 8 - sz;
+}
+
+// intersectBoundT (Util.cl:707-732) on near and far planes.  EXACT: the
+// reference's chain of conditional assignments, as box_hit.  Otherwise, for
+// plain rays: the conjunction of its early outs is max(near) <= min(far) (the
+// same-axis pairs hold by themselves), and its t is max(near).
+template <bool EXACT>
+__device__ __forceinline__ bool slab(const WaveRay& R, float nx, float ny, float nz, float fx, float fy, float fz,
+                                     float& tnear)
+{
+    const float tmin = (nx - R.o.x) * R.inv.x, tmax = (fx - R.o.x) * R.inv.x;
+    const float tymin = (ny - R.o.y) * R.inv.y, tymax = (fy - R.o.y) * R.inv.y;
+    const float tzmin = (nz - R.o.z) * R.inv.z, tzmax = (fz - R.o.z) * R.inv.z;
+    if (EXACT) {
+        const bool xy = !((tmin > tymax) | (tymin > tmax));
+        const float t1 = tymin > tmin ? tymin : tmin;
+        const float u1 = tymax < tmax ? tymax : tmax;
+        const bool xyz = !((t1 > tzmax) | (tzmin > u1));
+        const float t2 = tzmin > t1 ? tzmin : t1;
+        const float u2 = (tzmax < u1 ? tzmax : u1) * 1.00000024f;
+        tnear = t2;
+        return xy & xyz & (t2 < R.tmax) & (u2 > R.tmin);
+    }
+    const float t2 = fmaxf(fmaxf(tmin, tymin), tzmin), u = fminf(fminf(tmax, tymax), tzmax);
+    tnear = t2;
+    return (t2 <= u) & (t2 < R.tmax) & (u * 1.00000024f > R.tmin);
+}
+
+// A lane's pending subtrees lie in its column of the LDS stack, oldest first,
+// above a row that holds WT_NONE (popped when none is left); those past the
+// column's last row lie in `ovf`.  sp is the address of the row above the newest
+// (256 bytes per row), `last` the address past the column.
+__device__ __forceinline__ int wave_top(int sp, int last, const int* ovf)
+{
+    if (__any(sp > last)) { // rare
+        if (sp > last) return ovf[(((sp - last) >> 8) - 1) & (WT_OVF - 1)];
+    }
+    return lds_word(sp - 256);
+}
+
+// One interior node for every lane that holds one.  Called with the whole
+// wave active.
+template <bool EXACT, bool WIDE, bool STAGED>
+__device__ __forceinline__ void wave_step(const char* __restrict__ nodes, lds_char* slots, int last, int c16,
+                                          int slot, WaveRay& R, int* ovf)
+{
+    const bool inner = R.cur >= 0;
+    const int node = inner ? R.cur : 0; // the other lanes load the root's record
+    vf2 nx, ny, nz, fx, fy, fz;
+    vi2 ref;
+    float4 px, py, pz;
+    if (STAGED) {
+        int alo, ahi = 0;
+        if (WIDE) { // 64-bit address of this lane's node
+            const uint64_t a = reinterpret_cast<uint64_t>(nodes) + ((uint64_t)(uint32_t)node << 6);
+            alo = (int)(uint32_t)a;
+            ahi = (int)(uint32_t)(a >> 32);
+        } else {
+            alo = node << 6; // byte offset into the scene's records
+        }
+#define WT_LOAD(J)                                                                                                   \
+    {                                                                                                                \
+        const char* a_;                                                                                              \
+        if (WIDE)                                                                                                    \
+            a_ = reinterpret_cast<const char*>(((uint64_t)(uint32_t)quad_bcast<J>(ahi) << 32) |                      \
+                                               (uint32_t)quad_bcast<J>(alo)) + c16;                                  \
+        else a_ = nodes + (uint32_t)(quad_bcast<J>(alo) + c16);                                                      \
+        __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)a_,                          \
+                                         (__attribute__((address_space(3))) void*)(slots + J * WT_SLOT), 16, 0, 0); \
+    }
+        WT_LOAD(0)
+        WT_LOAD(1)
+        WT_LOAD(2)
+        WT_LOAD(3)
+#undef WT_LOAD
+    } else {
+        const char* N = WIDE ? nodes + ((uint64_t)(uint32_t)node << 6) : nodes + (uint32_t)(node << 6);
+        px = *reinterpret_cast<const float4*>(N);
+        py = *reinterpret_cast<const float4*>(N + 16);
+        pz = *reinterpret_cast<const float4*>(N + 32);
+        ref = *reinterpret_cast<const vi2*>(N + 48);
+    }
+    const bool deep = __any(R.sp >= last); // rare
+    int top;
+    if (deep && R.sp > last) top = ovf[(((R.sp - last) >> 8) - 1) & (WT_OVF - 1)];
+    else top = lds_word(R.sp - 256);
+    if (STAGED) {
+        __builtin_amdgcn_s_waitcnt(0x0f70); // vmcnt(0): the records are in LDS
+        nx = lds_pair(R.nx), fx = lds_pair(R.fx);
+        ny = lds_pair(R.ny + 16), fy = lds_pair(R.fy + 16);
+        nz = lds_pair(R.nz + 32), fz = lds_pair(R.fz + 32);
+        ref = *(__attribute__((address_space(3))) vi2*)(slot + 48);
+    } else {
+        auto pick = [](int neg, float4 p, vf2& n, vf2& f) {
+            n.x = neg ? p.z : p.x, n.y = neg ? p.w : p.y;
+            f.x = neg ? p.x : p.z, f.y = neg ? p.y : p.w;
+        };
+        pick(R.nx, px, nx, fx);
+        pick(R.ny, py, ny, fy);
+        pick(R.nz, pz, nz, fz);
+    }
+    float lt, rt;
+    const bool lh = inner && slab<EXACT>(R, nx.x, ny.x, nz.x, fx.x, fy.x, fz.x, lt);
+    const bool rh = inner && slab<EXACT>(R, nx.y, ny.y, nz.y, fx.y, fy.y, fz.y, rt);
+    const bool both = lh && rh;
+    const bool right = rh && (!lh || rt < lt); // nearer child first, ties to the left
+    const bool pop = inner && !lh && !rh;
+    const int near = right ? ref.y : ref.x, far = right ? ref.x : ref.y;
+    if (deep) {
+        if (both && R.sp >= last) ovf[((R.sp - last) >> 8) & (WT_OVF - 1)] = far;
+        else if (both) lds_word(R.sp) = far;
+    } else {
+        lds_word(R.sp) = far; // above the top: kept only where both were hit
+    }
+    R.cur = pop ? top : (inner ? near : R.cur);
+    R.sp += both ? 256 : 0;
+    R.sp -= pop ? 256 : 0;
+}
+
+// Traces the rays of entries [next, end) (wave-uniform).  load(id, r, sc)
+// fills entry id's ray (WIDE: and may set the lane's scene, whose records are then
+// addressed with 64 bits); done(fin, id, t, child, sc) is called with the whole
+// wave active, fin set on the lanes whose ray has ended (t: its tMax after the
+// walk, child: the leaf hit or WT_NONE).  `wave_lds`: one per wave of the
+// work-group.
+template <bool ANY, bool WIDE, int REFILL, WaveForm F, class Load, class Done>
+__device__ __forceinline__ void wave_trace(WaveLds<F>* wave_lds, MtSceneRef scene, int next, int end, Load&& load,
+                                           Done&& done)
+{
+    constexpr bool STAGED = F != WT_DIRECT;
+    const int lane = __lane_id();
+    WaveLds<F>* lds = wave_lds + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    lds_char* slots = (lds_char*)lds->node;
+    const int slot = STAGED ? (int)(uintptr_t)slots + (lane & 3) * WT_SLOT + (lane >> 2) * 64 : 0;
+    const int col = (int)(uintptr_t)(lds_int*)&lds->stack[0][lane];
+    const int last = col + 256 * (WaveLds<F>::ROWS + 1);
+    const int c16 = (lane & 3) << 4;
+    int ovf[WT_OVF];
+    bool active = false, ended = false, plain = true;
     int id = 0;
-    RayT r;
-    TravStateN<N> S;
-    const float4* lpn = pn; // this lane's scene (load may change it)
-    const float4* lpt = pt;
-    int lroot = root;
+    MtSceneRef sc = scene; // this lane's scene
+    WaveRay R;
+    R.cur = WT_NONE;
+    R.sp = col + 256;
+    R.nx = R.ny = R.nz = R.fx = R.fy = R.fz = slot;
     for (;;) {
         const uint64_t idle = __ballot(!active);
-        // refill once POOL_REFILL_MIN lanes wait (or all do): starting a ray
-        // (two loads, three reciprocals) for one or two lanes at a time would
-        // cost the whole wave that block nearly every iteration
-        if (idle && next < end && (idle == ~0ull || __popcll(idle) >= POOL_REFILL_MIN)) {
-            const int avail = end - next, nidle = (int)__popcll(idle);
+        const int nidle = (int)__popcll(idle);
+        if (nidle == 64 || (next < end && nidle >= REFILL)) {
+            if (__any(ended)) done(ended, id, R.tmax, R.child, sc);
+            ended = false;
+            if (next >= end) break; // run drained, every lane done
+            const int avail = end - next;
             const int n = avail < nidle ? avail : nidle;
             const int rk = (int)lane_rank(idle);
             if (!active && rk < n) {
                 id = next + rk;
-                load(id, r, lpn, lpt, lroot);
-                S.init(lroot);
+                RayT r;
+                load(id, r, sc);
+                wave_ray_start(R, r, slot, col, sc.root);
+                plain = ray_plain(r) && sc.plain;
                 active = true;
             }
             next += n;
         }
-        if (!__any(active)) break; // run drained, every lane done
-        bool fin = false;
-        if (active && trace_packed_node<ANY, false>(lpn, lpt, r, S)) {
-            fin = true;
-            active = false;
+        const int thr = (int)__popcll(__ballot(active)) * 3 / 4;
+        const char* nodes = reinterpret_cast<const char*>(WIDE ? sc.pn : scene.pn);
+        if (__any(active && !plain)) {
+            while ((int)__popcll(__ballot(R.cur >= 0)) > thr)
+                wave_step<true, WIDE, STAGED>(nodes, slots, last, c16, slot, R, ovf);
+        } else {
+            while ((int)__popcll(__ballot(R.cur >= 0)) > thr)
+                wave_step<false, WIDE, STAGED>(nodes, slots, last, c16, slot, R, ovf);
         }
-        done(fin, id, r, S);
+        if (R.cur < 0 && R.cur != WT_NONE) {
+            const float4* T = (WIDE ? sc.pt : scene.pt) + 3 * (size_t)(~R.cur);
+            const float4 t0 = T[0], t1 = T[1];
+            const float e2z = T[2].x;
+            RayT r;
+            r.o = R.o;
+            r.d = R.d;
+            r.tmax = R.tmax;
+            const float t = tri_hit(r, mk3(t0.x, t0.y, t0.z), mk3(t0.w, t1.x, t1.y), mk3(t1.z, t1.w, e2z));
+            if ((R.tmin < t) && (t < R.tmax)) {
+                R.child = R.cur;
+                if (ANY) R.sp = col + 256; // found: nothing is pending any more
+                else R.tmax = t;
+            }
+            R.cur = wave_top(R.sp, last, ovf);
+            R.sp -= 256;
+        }
+        if (active && R.cur == WT_NONE) {
+            active = false;
+            ended = true;
+        }
     }
 }
 
-// The run of wave w of work-group b in a segmented queue (nseg segments of
-// seg_cap entries, counts[p] live in segment p) walked chunk-major with
-// runs of `run` entries: group v (seg_sweep_group) takes chunk v / nseg of
-// segment v % nseg, 4 runs, one per wave.
-__device__ __forceinline__ void pool_seg_run(const int* __restrict__ counts, int nseg, int seg_cap, int run,
-                                             int& next, int& end)
+// Primitive of a leaf, -1 for none.
+__device__ __forceinline__ int leaf_prim(const float4* __restrict__ pt, int child)
+{
+    return child != WT_NONE ? __float_as_int(pt[3 * (size_t)(~child) + 2].y) : -1;
+}
+
+// How a launch is split into waves: a wave takes `run` consecutive rays, so
+// many that the launch just fills the GPU's wave slots (`slots`, of the
+// kernel's form) where there are few rays, WT_MAX_RUN where there are many (a
+// wave's start and drain, with few lanes busy, then weigh little).  993K soup
+// rays per bounce: filling exactly the staged form's 6144 slots instead of
+// 8192 waves took a whole render from 5.49 to 5.07 ms (the last third of a
+// second round of waves is gone); 957K short rays in runs of 30 instead of
+// 128: 0.29 -> 0.73 ms.
+
+// Rays per wave of a plain queue of up to n entries.
+inline int wave_run(int64_t n, int slots)
+{
+    const int64_t r = (n / slots + 15) & ~(int64_t)15;
+    return (int)(r < WT_MIN_RUN ? WT_MIN_RUN : (r > WT_MAX_RUN ? WT_MAX_RUN : r));
+}
+
+// Work-groups per segment of a queue of nseg segments.
+inline int wave_seg_groups(int seg_cap, int nseg, int slots)
+{
+    const int want = slots / 4 / nseg;
+    const int full = (seg_cap + 4 * WT_MAX_RUN - 1) / (4 * WT_MAX_RUN);
+    const int most = (seg_cap + 4 * WT_MIN_RUN - 1) / (4 * WT_MIN_RUN);
+    return full > want ? full : (want < most ? want : most);
+}
+
+// The run of this wave in a queue of nseg segments of seg_cap entries,
+// counts[p] live in segment p: work-group v (seg_sweep_group) belongs to
+// segment v mod nseg.  Lengths as above, from the segment's count.
+__device__ __forceinline__ void seg_run(const int* __restrict__ counts, int nseg, int seg_cap, int slots, int& next,
+                                        int& end)
 {
     const unsigned v = seg_sweep_group();
     const int p = (int)(v % (unsigned)nseg), c = (int)(v / (unsigned)nseg);
+    const int waves = (int)(gridDim.x / (unsigned)nseg) * 4;
     int cnt = counts[p];
     cnt = cnt < seg_cap ? cnt : seg_cap;
-    const int off = c * (4 * run) + (int)(threadIdx.x >> 6) * run;
+    const int want = slots / nseg;
+    int run = (cnt + want - 1) / want;
+    run = run < WT_MIN_RUN ? WT_MIN_RUN : (run > WT_MAX_RUN ? WT_MAX_RUN : run);
+    if (run < (cnt + waves - 1) / waves) run = (cnt + waves - 1) / waves; // the grid covers the segment
+    const int off = (c * 4 + (int)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6)) * run;
     next = p * seg_cap + off;
     end = p * seg_cap + (cnt < off + run ? cnt : off + run);
 }
 
-// Rays per lane of a wave's run in the pool kernels.
-constexpr int POOL_RAYS = 4;
-// Short-stack depth of the wave pools over sorted (binned) batches: a deep
-// tree's rays keep more postponed subtrees in registers (64M random rays
-// through 4M triangles, depth 45: see mt_trace.hip).
-constexpr int SHORT_STACK_DEEP = 12;
+// Whether node records lie beyond a 32-bit byte offset.
+inline bool scene_wide(const mt_scene* sc) { return sc->num_interior > (1 << 26); }
 
 template <bool ANY, bool STATS, bool SHORT_STACK>
 __device__ __forceinline__ int trace_packed(const float4* __restrict__ pn,
@@ -511,8 +676,8 @@ __device__ __forceinline__ int trace_packed(const float4* __restrict__ pn,
             float4 a = N[0], b = N[1], c = N[2];
             int4 d = *reinterpret_cast<const int4*>(N + 3);
             float lt, rt;
-            bool lh = box_hit(r, a.x, a.y, a.z, a.w, b.x, b.y, lt);
-            bool rh = box_hit(r, b.z, b.w, c.x, c.y, c.z, c.w, rt);
+            bool lh = box_hit(r, a.x, b.x, c.x, a.z, b.z, c.z, lt);
+            bool rh = box_hit(r, a.y, b.y, c.y, a.w, b.w, c.w, rt);
             if (STATS) st[0]++;
             if (!lh && !rh) break;
             bs.push0();
