@@ -176,8 +176,8 @@ typedef struct {
 /* CNormalBVH.build (CNormalBVH.java:45-148) on the device: from device
  * points/faces (layout above) into device nodes/bounds, the same tree as
  * mt_bvh_build (node numbering, leaf primitives, bounds; a zero bound may
- * differ in sign).  Builds one level of the tree per round and reads each
- * round's node count back, so the call synchronises the context's stream.
+ * differ in sign).  Synchronises the context's stream (it reads node counts
+ * back every few levels).
  * max_depth (host) receives the deepest leaf (root = 0). */
 int32_t mt_bvh_build_device(mt_context* ctx, int32_t ntris, const float* points,
                             const int32_t* faces, int32_t* nodes, float* bounds,

@@ -30,7 +30,7 @@
 // callers expect (PrefixSumIntegerTest.java:30-36, LightConfiguration.cl:
 // 31-55).  CompactAtomic's order is whatever its atomic_inc produces; this
 // compaction is stable (survivors in index order), matching prepareLightInfo.
-#include "mt_internal.h"
+#include "mt_lookback.h"
 
 #include <mutex>
 
@@ -40,13 +40,6 @@ constexpr int SCAN_THREADS = 256;
 constexpr int SCAN_ROWS = 32;
 constexpr int SCAN_TILE = SCAN_THREADS * SCAN_ROWS;
 constexpr int SCAN_WAVES = SCAN_THREADS / 64;
-constexpr uint32_t FLAG_AGG = 1u, FLAG_INC = 2u;
-constexpr uint32_t SPIN_LIMIT = 1u << 26;
-
-struct ScanWork {
-    uint32_t* ticket; // [0] ticket, [1] error flag (spin limit hit), [2] epoch of the current call
-    uint64_t* status; // [ntiles]
-};
 
 // Tile I/O goes through buffer resources ("windows"): a descriptor whose
 // range check drops stores and zeroes loads at byte offsets at or past its
@@ -79,73 +72,6 @@ template <> struct BufIO<16> {
     static __device__ T ld(__amdgpu_buffer_rsrc_t r, uint32_t o) { return __builtin_amdgcn_raw_buffer_load_b128(r, o, 0, 0); }
     static __device__ void st(T v, __amdgpu_buffer_rsrc_t r, uint32_t o) { __builtin_amdgcn_raw_buffer_store_b128(v, r, o, 0, 0); }
 };
-
-__device__ __forceinline__ uint64_t pack_status(uint32_t epoch, uint32_t flag, uint32_t v)
-{
-    return ((uint64_t)(epoch & 0x3FFFFFFFu) << 34) | ((uint64_t)flag << 32) | (uint64_t)v;
-}
-
-__device__ __forceinline__ int lane_id() { return __lane_id(); }
-
-__device__ __forceinline__ uint32_t lane_rank(uint64_t mask)
-{ // number of set bits of `mask` below this lane (v_mbcnt_lo/hi)
-    return __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
-}
-
-// Decoupled look-back by wave 0 of the tile.  Returns the exclusive prefix of
-// `tile` (all lanes of wave 0 agree); publishes the tile's inclusive prefix.
-__device__ uint32_t look_back(ScanWork W, int tile, uint32_t aggregate, uint32_t epoch)
-{
-    const int lane = lane_id();
-    uint64_t* st = W.status;
-    if (tile == 0) {
-        if (lane == 0)
-            __hip_atomic_store(&st[0], pack_status(epoch, FLAG_INC, aggregate), __ATOMIC_RELAXED,
-                               __HIP_MEMORY_SCOPE_AGENT);
-        return 0u;
-    }
-    if (lane == 0)
-        __hip_atomic_store(&st[tile], pack_status(epoch, FLAG_AGG, aggregate), __ATOMIC_RELAXED,
-                           __HIP_MEMORY_SCOPE_AGENT);
-    uint32_t prefix = 0;
-    int window_end = tile - 1; // predecessor examined by lane 0
-    const uint32_t ep = epoch & 0x3FFFFFFFu;
-    uint32_t spins = 0;
-    for (;;) {
-        int idx = window_end - lane;
-        uint64_t w;
-        uint32_t flag, val;
-        for (;;) {
-            if (idx >= 0) {
-                w = __hip_atomic_load(&st[idx], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                bool cur = (uint32_t)(w >> 34) == ep;
-                flag = cur ? (uint32_t)(w >> 32) & 3u : 0u;
-                val = (uint32_t)w;
-            } else { // before tile 0: an inclusive zero
-                flag = FLAG_INC;
-                val = 0;
-            }
-            if (__all(flag != 0)) break;
-            if (++spins > SPIN_LIMIT) {
-                if (lane == 0) atomicOr(&W.ticket[1], 1u);
-                return prefix; // results invalid; the host reports the error flag
-            }
-            __builtin_amdgcn_s_sleep(1);
-        }
-        uint64_t inc = __ballot(flag == FLAG_INC);
-        // lanes up to and including the nearest inclusive predecessor contribute
-        int first_inc = inc ? __builtin_ctzll(inc) : 64;
-        uint32_t contrib = lane <= first_inc ? val : 0u;
-        for (int o = 32; o > 0; o >>= 1) contrib += __shfl_xor(contrib, o);
-        prefix += contrib;
-        if (inc) break;
-        window_end -= 64;
-    }
-    if (lane == 0)
-        __hip_atomic_store(&st[tile], pack_status(epoch, FLAG_INC, prefix + aggregate),
-                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    return prefix;
-}
 
 __global__ void k_scan_reset(ScanWork W, const int* __restrict__ d_len, int capacity,
                              int* __restrict__ d_total)
@@ -450,17 +376,6 @@ __global__ void k_isects_finish(float4* __restrict__ isects, int* __restrict__ p
         if (q == 5) pixels[j] = 0;
     }
     isects[i] = v;
-}
-
-int32_t scan_workspace_tiles(mt_context* ctx, int64_t ntiles, ScanWork& W)
-{
-    size_t bytes = 256 + sizeof(uint64_t) * (size_t)(ntiles > 0 ? ntiles : 1);
-    void* p = nullptr;
-    int32_t rc = mt_ctx_scratch(ctx, bytes, &p);
-    if (rc) return rc;
-    W.ticket = reinterpret_cast<uint32_t*>(p);
-    W.status = reinterpret_cast<uint64_t*>(reinterpret_cast<char*>(p) + 256);
-    return MT_OK;
 }
 
 int32_t scan_workspace(mt_context* ctx, int capacity, ScanWork& W)
