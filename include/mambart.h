@@ -535,7 +535,10 @@ typedef struct {
  * each late bounce's launches otherwise last as long as their slowest ray),
  * and costs when many do (the fused wavefront shares work across paths
  * better).  Applies to the default packed traversal modes without
- * MT_RENDER_TRAVERSAL_STATS; 0 (the default) or b >= max_bounces: off.  No
+ * MT_RENDER_TRAVERSAL_STATS; 0 (the default) or b >= max_bounces: off, except
+ * that a render of at most 262144 paths in mode MT_TRACE_PACKED or
+ * MT_TRACE_PACKED_STACK without MT_RENDER_PROFILE then runs all of its
+ * bounces in one such launch.  No
  * counterpart in the reference (its loop, CDeviceGI.java:214-271, launches
  * every stage of every bounce). */
 #define MT_RENDER_TAIL_SHIFT 8

@@ -300,66 +300,120 @@ __global__ __launch_bounds__(RT) void k_shade_split(ShadeArgs A, int* __restrict
     }
 }
 
-// Bounces tail..nb-1 of the fused loop in one launch (MT_RENDER_TAIL_FROM):
-// each lane takes a path of bounce `tail`'s segmented queue and carries it
+// Traces the rays (o, d) of the lanes with `have`, all to their end.
+template <bool ANY, bool WIDE>
+__device__ __forceinline__ void wave_all(const WaveLane<WT_DIRECT>& W, MtSceneRef scene, bool have, float4 o, float4 d,
+                                         WaveRay& R, int* ovf)
+{
+    bool active = have, plain = true;
+    if (have) {
+        RayT r;
+        ray_init(r, o, d);
+        wave_ray_start(R, r, W.slot, W.col, scene.root);
+        plain = ray_plain(r) && scene.plain;
+    }
+    const bool exact = __any(!plain);
+    while (__any(active)) wave_walk<ANY, WIDE>(W, scene, exact, R, active, ovf);
+}
+
+// Bounces of the fused loop in one launch: those from `tail` on
+// (MT_RENDER_TAIL_FROM), or all of a small render (WHOLE: path e is entry e,
+// its camera ray made in place).  Each lane takes a path and carries it
 // through all of its remaining bounces — closest hit, shading (shade_path),
-// shadow ray and its direct-light add — then takes its segment's next path.
-// Every path goes through the same operations in the same order as in the
-// per-bounce kernels (its radiance gains the shading's Ladd, then the
+// shadow ray and its direct-light add — then takes the next path of its
+// share.  Every path goes through the same operations in the same order as
+// in the per-bounce kernels (its radiance gains the shading's Ladd, then the
 // unoccluded shadow contribution, bounce after bounce; its random numbers
 // are keyed by (seed, path id, bounce); the light-grid sums are integers),
-// so the image and the grid are bit-identical.  What changes is the time
-// of the sparse late bounces: one launch whose length is the slowest path's
-// chain of dependent loads, instead of three launches per bounce, each as
-// long as that bounce's slowest ray.  Lanes of a wave stay in step (every
-// iteration is trace, shade, shadow for the lanes holding a path), only
-// their bounce numbers differ.  live[b] / shadow[b] count the paths
-// entering bounce b > tail and the shadow rays of bounce b >= tail (the
-// per-bounce kernels' queue lengths), summed in LDS, one atomic per
-// work-group and bounce.
-constexpr int TAIL_SWEEP = 8; // work-groups per segment
-__global__ __launch_bounds__(RT) void k_tail(ShadeArgs A, const float4* __restrict__ pn,
-                                             const float4* __restrict__ pt, int root, int nb,
-                                             int* __restrict__ live_out, int* __restrict__ shadow_out)
+// so the image and the grid are bit-identical.  What changes is the time of
+// sparse bounces: one launch whose length is the slowest path's chain of
+// dependent loads, instead of three launches per bounce, each as long as
+// that bounce's slowest ray.  Lanes of a wave stay in step (every iteration
+// is trace, shade, shadow for the lanes holding a path), only their bounce
+// numbers differ.  live[b] / shadow[b] count the paths entering bounce b >
+// tail and the shadow rays of bounce b >= tail (the per-bounce kernels'
+// queue lengths), summed in LDS, one atomic per work-group and bounce.
+//
+// What bounds it: the dependent node loads of one wave's lanes, so a wave is
+// given few lanes where the chip has wave slots to spare (`lanes`: 14400
+// soup paths, from bounce 1: 64 lanes a wave 968 us, 32 892, 16 857, 8 796;
+// 4096 paths in a closed room, all bounces: 8 907, 4 791, 2 733).  128
+// registers, four waves per SIMD: shade_path wants 172, and the spills cost
+// less than half the waves do (all bounces of 262144 soup paths: two waves
+// per SIMD 3.28 ms, three 3.11, four 2.35; 131072 paths in a room 1.42,
+// 1.41, 1.59; the late bounces of 33M paths on the open spheres 8.92, 8.84,
+// 8.74 ms the frame).  Its rays are traced as the per-bounce kernels trace
+// them (wave_walk); with one ray's loop after another per lane the same
+// 14400 paths took 1538 us from bounce 1.
+constexpr int TAIL_SWEEP = 16; // work-groups per segment
+constexpr int TAIL_MIN_LANES = 2;
+constexpr int TAIL_WAVES = 4; // per SIMD
+constexpr int TAIL_SLOTS = 1024 * TAIL_WAVES; // waves that the GPU's 1024 SIMDs hold at once
+// A render of at most so many paths runs as one launch: every path has a lane
+// at once.  Per-bounce launches (three each, ~12 us of gap, each as long as
+// its slowest ray) against it: 14400 soup paths 1078 -> 617 us, 16384 on open
+// spheres 502 -> 250, 4096 in a closed room 1305 -> 733, 131072 there 1773 ->
+// 1592, 262144 in the soup 3211 -> 2346, 240000 on spheres 696 -> 397.  Past
+// one round of lanes it loses: 524288 soup paths 3999 -> 3911, 993K 4.82 ->
+// 9.9 ms.
+constexpr int WHOLE_MAX = 64 * TAIL_SLOTS;
+template <bool WIDE, bool WHOLE>
+__global__ __launch_bounds__(RT, TAIL_WAVES) void k_tail(ShadeArgs A, MtSceneRef scene, int np, int nb, int lanes,
+                                                         int* __restrict__ counts, int* __restrict__ live_out,
+                                                         int* __restrict__ shadow_out)
 {
+    __shared__ WaveLds<WT_DIRECT> s_w[4];
     __shared__ int s_live[64], s_shadow[64];
+    const WaveLane<WT_DIRECT> W(s_w);
+    int ovf[WT_OVF];
+    WaveRay R;
+    W.idle(R);
     if (threadIdx.x < 64) {
         s_live[threadIdx.x] = 0;
         s_shadow[threadIdx.x] = 0;
     }
     __syncthreads();
     const uint32_t seed = *A.seed;
-    const int p = blockIdx.x % SHADOW_SEGS;
-    int cnt = A.in_seg[p];
-    cnt = cnt < A.seg_cap ? cnt : A.seg_cap;
-    const int stride = (int)(gridDim.x / SHADOW_SEGS) * (int)blockDim.x;
-    int e = (int)(blockIdx.x / SHADOW_SEGS) * (int)blockDim.x + (int)threadIdx.x; // this lane's next entry
+    const int p = WHOLE ? 0 : blockIdx.x % SHADOW_SEGS, groups = WHOLE ? gridDim.x : gridDim.x / SHADOW_SEGS;
+    int cnt = np;
+    if (!WHOLE) {
+        cnt = A.in_seg[p];
+        cnt = cnt < A.seg_cap ? cnt : A.seg_cap;
+    }
+    const int stride = groups * 4 * lanes, lane = __lane_id();
+    // this lane's next entry
+    int e = ((int)(WHOLE ? blockIdx.x : blockIdx.x / SHADOW_SEGS) * 4 + (int)(threadIdx.x >> 6)) * lanes + lane;
+    if (lane >= lanes) e = cnt;
+    if (WHOLE && blockIdx.x == 0 && threadIdx.x == 0) *counts = np;
     bool have = false;
     int pid = 0, b = 0;
     float4 ro = make_float4(0, 0, 0, 0), rd = ro, T4 = ro, L = ro;
     for (;;) {
         if (!have && e < cnt) { // refill: the next path of this lane's share of the segment
-            const int slot = p * A.seg_cap + e;
-            pid = A.queue[slot];
-            ro = A.o_tmin[slot];
-            rd = A.d_tmax[slot];
-            T4 = A.S.T[pid];
-            L = A.S.L[pid];
-            b = A.bounce;
+            if (WHOLE) {
+                pid = e;
+                const Camera C = A.C; // a register copy: a reference into the kernel argument spills it to scratch
+                camera_ray(C, pid, seed, ro, rd);
+                T4 = make_float4(1.0f, 1.0f, 1.0f, 1.0f);
+                L = make_float4(0, 0, 0, 0);
+                b = 0;
+            } else {
+                const int slot = p * A.seg_cap + e;
+                pid = A.queue[slot];
+                ro = A.o_tmin[slot];
+                rd = A.d_tmax[slot];
+                T4 = A.S.T[pid];
+                L = A.S.L[pid];
+                b = A.bounce;
+            }
             have = true;
             e += stride;
         }
         if (__ballot(have) == 0ull) break; // wave-uniform
-        int prim = -1;
-        float t = 0.0f;
-        if (have) { // closest hit, as k_trace_pool / k_trace_camera find it
-            RayT r;
-            ray_init(r, ro, rd);
-            int st[3] = {0, 0, 0};
-            int child = -1;
-            prim = trace_packed<false, false, true>(pn, pt, root, r, child, st) ? child : -1;
-            t = r.tmax;
-        }
+        // closest hit, as the per-bounce kernels find it
+        wave_all<false, WIDE>(W, scene, have, ro, rd, R, ovf);
+        const int prim = have ? leaf_prim(scene.pt, R.child) : -1;
+        const float t = R.tmax;
         PathOut P;
         P.has_shadow = false;
         P.alive = false;
@@ -371,16 +425,11 @@ __global__ __launch_bounds__(RT) void k_tail(ShadeArgs A, const float4* __restri
                 L = make_float4(L.x + P.Ladd.x, L.y + P.Ladd.y, L.z + P.Ladd.z, L.w);
         }
         if (A.V.G.mode) lg_wave_accum(P.acc_gidx >= 0, P.acc_gidx, P.acc_q, A.V.G.pend); // whole wave active
-        bool vis = false;
-        if (P.has_shadow) { // any hit; an unoccluded sample adds its contribution
-            atomicAdd(&s_shadow[b], 1);
-            RayT r;
-            ray_init(r, P.so, P.sd);
-            int st[3] = {0, 0, 0};
-            int child = -1;
-            vis = !trace_packed<true, false, true>(pn, pt, root, r, child, st);
-            if (vis) L = make_float4(L.x + P.contrib.x, L.y + P.contrib.y, L.z + P.contrib.z, L.w);
-        }
+        // any hit; an unoccluded sample adds its contribution
+        if (P.has_shadow) atomicAdd(&s_shadow[b], 1);
+        wave_all<true, WIDE>(W, scene, P.has_shadow, P.so, P.sd, R, ovf);
+        const bool vis = P.has_shadow && R.child == WT_NONE;
+        if (vis) L = make_float4(L.x + P.contrib.x, L.y + P.contrib.y, L.z + P.contrib.z, L.w);
         if (A.V.G.mode && A.V.G.pend)
             lg_wave_accum(vis && P.shadow_gidx >= 0, P.shadow_gidx, lg_fixed(P.shadow_lum), A.V.G.pend);
         if (have) {
@@ -483,7 +532,7 @@ struct RenderPlan {
         oIlp, oTot, oSeed, oSlg, oHit, oHsc, oTail;
     mt_lightgrid* grid; // guided environment mode: the grid the render samples and accumulates into
     bool fused; // camera rays traced in place, shadow adds fused, next queue appended by the shading stage
-    int tail;   // fused loop: bounces tail..nb-1 run in one k_tail launch (0: none)
+    int tail;   // fused loop: bounces tail..nb-1 run in one k_tail launch (0: the whole render; -1: none)
     bool borrowed; // base is the context's reusable workspace (mt_render), not owned
     hipEvent_t ev[4 * 64];
     int nev;
@@ -574,8 +623,13 @@ int32_t plan_render(const mt_scene* scene, const float* materials, const mt_envm
     R.fused = (desc->mode == MT_TRACE_PACKED || desc->mode == MT_TRACE_PACKED_STACK ||
                desc->mode == MT_TRACE_PACKED_SORTED || desc->mode == MT_TRACE_PACKED_POOL) && !R.want_ilp;
     R.tail = (desc->flags >> MT_RENDER_TAIL_SHIFT) & 63;
-    if (!R.fused || R.tail >= R.nb) R.tail = 0; // the tail applies to the fused loop's bounces >= 1
     R.profile = (desc->flags & MT_RENDER_PROFILE) != 0;
+    if (!R.fused || R.tail == 0 || R.tail >= R.nb) R.tail = -1; // the tail applies to the fused loop's bounces >= 1
+    // a small render of the default traversal: all bounces in one launch (the
+    // profile's per-stage times need the stages)
+    if (R.tail < 0 && R.fused && (desc->mode == MT_TRACE_PACKED || desc->mode == MT_TRACE_PACKED_STACK) &&
+        !R.profile && R.np <= WHOLE_MAX)
+        R.tail = 0;
     R.oIlp = R.want_ilp ? take(12 * (R.sq > n ? R.sq : n)) : 0;
     R.oTot = take(8 * 8 * ILP_SLOTS);
     R.oSeed = take(4);
@@ -673,7 +727,11 @@ int32_t enqueue_render(mt_context* ctx, RenderPlan& R)
     // extra groups could never find work, only be dispatched)
     const int seg_chunks = (int)(((int64_t)seg_cap + RT - 1) / RT);
     const int gsweep = SHADOW_SEGS * (seg_chunks < SEG_SWEEP ? seg_chunks : SEG_SWEEP);
-    const int gtail = SHADOW_SEGS * (seg_chunks < TAIL_SWEEP ? seg_chunks : TAIL_SWEEP);
+    int tail_lanes = TAIL_MIN_LANES; // paths a wave of k_tail holds at a time
+    while (tail_lanes < 64 && (int64_t)TAIL_SLOTS * tail_lanes < np) tail_lanes *= 2;
+    const int tail_groups = (seg_cap + 4 * tail_lanes - 1) / (4 * tail_lanes);
+    const int gtail = SHADOW_SEGS * (tail_groups < TAIL_SWEEP ? tail_groups : TAIL_SWEEP);
+    const int gwhole = mt_blocks(np, 4 * tail_lanes); // at most TAIL_SLOTS / 4: np <= WHOLE_MAX
     const MtSceneRef sref{scene->pnodes, scene->ptris, scene->root_ref, scene->plain};
     const bool wide = scene_wide(scene);
     const int cam_run = wave_run(np, WaveLds<WT_DIRECT>::SLOTS);
@@ -761,10 +819,12 @@ int32_t enqueue_render(mt_context* ctx, RenderPlan& R)
     for (int b = 0; b < nb && rc == MT_OK; b++) {
         int* dcount = counts + b;
         const bool first = fused && b == 0;
-        if (R.tail && b == R.tail) { // every remaining bounce in one launch
+        if (b == R.tail) { // every remaining bounce in one launch
             if ((rc = join_pending())) break;
-            k_tail<<<gtail, RT, 0, st>>>(shade_args(b, false), scene->pnodes, scene->ptris,
-                                                          scene->root_ref, nb, I(R.oTail), I(R.oTail) + 64);
+            auto kern = b == 0 ? (wide ? k_tail<true, true> : k_tail<false, true>)
+                               : (wide ? k_tail<true, false> : k_tail<false, false>);
+            kern<<<b == 0 ? gwhole : gtail, RT, 0, st>>>(shade_args(b, b == 0), sref, np, nb, tail_lanes, counts,
+                                                         I(R.oTail), I(R.oTail) + 64);
             rc = chk();
             break;
         }
@@ -895,7 +955,7 @@ int32_t read_stats(mt_context* ctx, RenderPlan& R, mt_render_stats* stats)
             hc[b] = (int)c;
         }
     }
-    if (R.tail) { // k_tail's bounces: paths entering bounces > tail, shadow rays of bounces >= tail
+    if (R.tail >= 0) { // k_tail's bounces: paths entering bounces > tail, shadow rays of bounces >= tail
         int tl[128];
         e = hipMemcpyAsync(tl, R.base + R.oTail, sizeof(tl), hipMemcpyDeviceToHost, st);
         if (e == hipSuccess) e = hipStreamSynchronize(st);
@@ -919,7 +979,7 @@ int32_t read_stats(mt_context* ctx, RenderPlan& R, mt_render_stats* stats)
     stats->closest_launches = stats->any_launches = 0;
     stats->closest_ms = stats->any_ms = 0.0f;
     if (R.profile) {
-        for (int b = 0; b < (R.tail ? R.tail : nb); b++) { // k_tail's bounces have no per-stage events
+        for (int b = 0; b < (R.tail >= 0 ? R.tail : nb); b++) { // k_tail's bounces have no per-stage events
             float ms = 0.0f;
             if (hipEventElapsedTime(&ms, R.ev[4 * b], R.ev[4 * b + 1]) == hipSuccess) {
                 stats->closest_ms += ms;

@@ -527,6 +527,68 @@ __device__ __forceinline__ void wave_step(const char* __restrict__ nodes, lds_ch
     R.sp -= pop ? 256 : 0;
 }
 
+// What a wave's lanes need besides their rays.
+template <WaveForm F>
+struct WaveLane {
+    lds_char* slots;
+    int slot, col, last, c16;
+    __device__ __forceinline__ WaveLane(WaveLds<F>* wave_lds)
+    {
+        const int lane = __lane_id();
+        WaveLds<F>* lds = wave_lds + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+        slots = (lds_char*)lds->node;
+        slot = F != WT_DIRECT ? (int)(uintptr_t)slots + (lane & 3) * WT_SLOT + (lane >> 2) * 64 : 0;
+        col = (int)(uintptr_t)(lds_int*)&lds->stack[0][lane];
+        last = col + 256 * (WaveLds<F>::ROWS + 1);
+        c16 = (lane & 3) << 4;
+    }
+    __device__ __forceinline__ void idle(WaveRay& R) const
+    { // a lane that has had no ray yet
+        R.cur = WT_NONE;
+        R.sp = col + 256;
+        R.nx = R.ny = R.nz = R.fx = R.fy = R.fz = slot;
+    }
+};
+
+// Takes the wave's rays (lanes with `active`) on until leaves have been tested once:
+// interior nodes while more than three quarters of the rays are at one, then the
+// leaves that have been reached.  Clears `active` where a ray has ended.
+// exact: some active ray needs intersectBoundT's chain.  Called with the whole
+// wave active.
+template <bool ANY, bool WIDE, WaveForm F>
+__device__ __forceinline__ void wave_walk(const WaveLane<F>& W, MtSceneRef sc, bool exact, WaveRay& R, bool& active,
+                                          int* ovf)
+{
+    constexpr bool STAGED = F != WT_DIRECT;
+    const int thr = (int)__popcll(__ballot(active)) * 3 / 4;
+    const char* nodes = reinterpret_cast<const char*>(sc.pn);
+    if (exact) {
+        while ((int)__popcll(__ballot(R.cur >= 0)) > thr)
+            wave_step<true, WIDE, STAGED>(nodes, W.slots, W.last, W.c16, W.slot, R, ovf);
+    } else {
+        while ((int)__popcll(__ballot(R.cur >= 0)) > thr)
+            wave_step<false, WIDE, STAGED>(nodes, W.slots, W.last, W.c16, W.slot, R, ovf);
+    }
+    if (R.cur < 0 && R.cur != WT_NONE) {
+        const float4* T = sc.pt + 3 * (size_t)(~R.cur);
+        const float4 t0 = T[0], t1 = T[1];
+        const float e2z = T[2].x;
+        RayT r;
+        r.o = R.o;
+        r.d = R.d;
+        r.tmax = R.tmax;
+        const float t = tri_hit(r, mk3(t0.x, t0.y, t0.z), mk3(t0.w, t1.x, t1.y), mk3(t1.z, t1.w, e2z));
+        if ((R.tmin < t) && (t < R.tmax)) {
+            R.child = R.cur;
+            if (ANY) R.sp = W.col + 256; // found: nothing is pending any more
+            else R.tmax = t;
+        }
+        R.cur = wave_top(R.sp, W.last, ovf);
+        R.sp -= 256;
+    }
+    if (R.cur == WT_NONE) active = false;
+}
+
 // Traces the rays of entries [next, end) (wave-uniform).  load(id, r, sc)
 // fills entry id's ray (WIDE: and may set the lane's scene, whose records are then
 // addressed with 64 bits); done(fin, id, t, child, sc) is called with the whole
@@ -537,26 +599,18 @@ template <bool ANY, bool WIDE, int REFILL, WaveForm F, class Load, class Done>
 __device__ __forceinline__ void wave_trace(WaveLds<F>* wave_lds, MtSceneRef scene, int next, int end, Load&& load,
                                            Done&& done)
 {
-    constexpr bool STAGED = F != WT_DIRECT;
-    const int lane = __lane_id();
-    WaveLds<F>* lds = wave_lds + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    lds_char* slots = (lds_char*)lds->node;
-    const int slot = STAGED ? (int)(uintptr_t)slots + (lane & 3) * WT_SLOT + (lane >> 2) * 64 : 0;
-    const int col = (int)(uintptr_t)(lds_int*)&lds->stack[0][lane];
-    const int last = col + 256 * (WaveLds<F>::ROWS + 1);
-    const int c16 = (lane & 3) << 4;
+    const WaveLane<F> W(wave_lds);
     int ovf[WT_OVF];
     bool active = false, ended = false, plain = true;
     int id = 0;
     MtSceneRef sc = scene; // this lane's scene
     WaveRay R;
-    R.cur = WT_NONE;
-    R.sp = col + 256;
-    R.nx = R.ny = R.nz = R.fx = R.fy = R.fz = slot;
+    W.idle(R);
     for (;;) {
         const uint64_t idle = __ballot(!active);
         const int nidle = (int)__popcll(idle);
         if (nidle == 64 || (next < end && nidle >= REFILL)) {
+            ended = ended && !active;
             if (__any(ended)) done(ended, id, R.tmax, R.child, sc);
             ended = false;
             if (next >= end) break; // run drained, every lane done
@@ -567,42 +621,14 @@ __device__ __forceinline__ void wave_trace(WaveLds<F>* wave_lds, MtSceneRef scen
                 id = next + rk;
                 RayT r;
                 load(id, r, sc);
-                wave_ray_start(R, r, slot, col, sc.root);
+                wave_ray_start(R, r, W.slot, W.col, sc.root);
                 plain = ray_plain(r) && sc.plain;
                 active = true;
             }
             next += n;
         }
-        const int thr = (int)__popcll(__ballot(active)) * 3 / 4;
-        const char* nodes = reinterpret_cast<const char*>(WIDE ? sc.pn : scene.pn);
-        if (__any(active && !plain)) {
-            while ((int)__popcll(__ballot(R.cur >= 0)) > thr)
-                wave_step<true, WIDE, STAGED>(nodes, slots, last, c16, slot, R, ovf);
-        } else {
-            while ((int)__popcll(__ballot(R.cur >= 0)) > thr)
-                wave_step<false, WIDE, STAGED>(nodes, slots, last, c16, slot, R, ovf);
-        }
-        if (R.cur < 0 && R.cur != WT_NONE) {
-            const float4* T = (WIDE ? sc.pt : scene.pt) + 3 * (size_t)(~R.cur);
-            const float4 t0 = T[0], t1 = T[1];
-            const float e2z = T[2].x;
-            RayT r;
-            r.o = R.o;
-            r.d = R.d;
-            r.tmax = R.tmax;
-            const float t = tri_hit(r, mk3(t0.x, t0.y, t0.z), mk3(t0.w, t1.x, t1.y), mk3(t1.z, t1.w, e2z));
-            if ((R.tmin < t) && (t < R.tmax)) {
-                R.child = R.cur;
-                if (ANY) R.sp = col + 256; // found: nothing is pending any more
-                else R.tmax = t;
-            }
-            R.cur = wave_top(R.sp, last, ovf);
-            R.sp -= 256;
-        }
-        if (active && R.cur == WT_NONE) {
-            active = false;
-            ended = true;
-        }
+        ended |= active;
+        wave_walk<ANY, WIDE>(W, WIDE ? sc : scene, __any(active && !plain), R, active, ovf);
     }
 }
 
@@ -621,11 +647,16 @@ __device__ __forceinline__ int leaf_prim(const float4* __restrict__ pt, int chil
 // second round of waves is gone); 957K short rays in runs of 30 instead of
 // 128: 0.29 -> 0.73 ms.
 
-// Rays per wave of a plain queue of up to n entries.
+// Rays per wave of a plain queue of up to n entries.  Below WT_MIN_RUN rays for
+// each of two waves per SIMD they are spread thinner: a wave lasts as long as
+// its lanes together need, but a wave of few lanes costs the SIMD as much as
+// a full one (with launch and read-back, 4096 camera rays in waves of 16: 278
+// us, of 4: 251; 30000 in waves of 16: 303, of 4: 391).
 inline int wave_run(int64_t n, int slots)
 {
-    const int64_t r = (n / slots + 15) & ~(int64_t)15;
-    return (int)(r < WT_MIN_RUN ? WT_MIN_RUN : (r > WT_MAX_RUN ? WT_MAX_RUN : r));
+    const int64_t r = (n / slots + 15) & ~(int64_t)15, few = (n / 2048 + 4) & ~(int64_t)3;
+    if (r <= WT_MIN_RUN) return (int)(few < WT_MIN_RUN ? few : WT_MIN_RUN);
+    return (int)(r > WT_MAX_RUN ? WT_MAX_RUN : r);
 }
 
 // Work-groups per segment of a queue of nseg segments.
