@@ -139,6 +139,19 @@ class Context:
     def scalar_i32(self, value: int):
         return _torch().tensor([value], dtype=_torch().int32, device=self.torch_device)
 
+    def _count(self, value: int):
+        """A device count for a launch of this context that follows at once: set
+        on the context's stream without waiting (scalar_i32 copies from
+        pageable memory and waits, a gap of 35 us before the launch).  When
+        torch's current stream is another one, whose allocator could hand
+        the word on too early, the copy that waits is kept."""
+        torch = _torch()
+        if torch.cuda.current_stream(self.torch_device).cuda_stream != self.stream.cuda_stream:
+            return self.scalar_i32(value)
+        out = torch.empty((1,), dtype=torch.int32, device=self.torch_device)
+        call("mt_buf_fill_i32", self.handle, _ptr(out), int(value), 1)
+        return out
+
 
 # ---------------------------------------------------------------------- host-side
 class CNormalBVH:
@@ -260,7 +273,7 @@ def intersect_primitives(ctx: Context, scene: Scene, o_tmin, d_tmax, count=None,
     _need(o_tmin, "o_tmin", n, (4,))
     _need(d_tmax, "d_tmax", n, (4,))
     if count is None:
-        count = ctx.scalar_i32(n)
+        count = ctx._count(n)
     prim = ctx.empty((n,), torch.int32)
     t = ctx.empty((n,), torch.float32)
     st = ctx.empty((n, 3), torch.int32) if stats else None
@@ -277,7 +290,7 @@ def intersect_occlusion(ctx: Context, scene: Scene, o_tmin, d_tmax, count=None, 
     _need(o_tmin, "o_tmin", n, (4,))
     _need(d_tmax, "d_tmax", n, (4,))
     if count is None:
-        count = ctx.scalar_i32(n)
+        count = ctx._count(n)
     occ = ctx.empty((n,), torch.int32)
     st = ctx.empty((n, 3), torch.int32) if stats else None
     call("mt_trace_any", ctx.handle, scene.handle, _ptr(o_tmin), _ptr(d_tmax), _ptr(count), n,
@@ -293,7 +306,7 @@ def autotune_trace(ctx: Context, scene: Scene, o_tmin, d_tmax, any_hit: bool = F
     _need(o_tmin, "o_tmin", n, (4,))
     _need(d_tmax, "d_tmax", n, (4,))
     if count is None:
-        count = ctx.scalar_i32(n)
+        count = ctx._count(n)
     prim = t = occ = None
     if any_hit:
         occ = ctx.empty((n,), torch.int32)
@@ -311,7 +324,7 @@ def shade_hits(ctx: Context, scene: Scene, o_tmin, d_tmax, prim, t, count=None):
     torch = _torch()
     n = o_tmin.shape[0]
     if count is None:
-        count = ctx.scalar_i32(n)
+        count = ctx._count(n)
     p = ctx.empty((n, 4), torch.float32)
     nn = ctx.empty((n, 4), torch.float32)
     ng = ctx.empty((n, 4), torch.float32)
@@ -354,7 +367,7 @@ def intersect_records(ctx: Context, scene: Scene, rays, isects, count=None, mode
     _need(isects, "isects", n, (INTERSECTION_RECORD_WORDS,), dtype=str(isects.dtype).split(".")[-1]
           if str(isects.dtype) in ("torch.int32", "torch.float32") else "float32")
     if count is None:
-        count = ctx.scalar_i32(n)
+        count = ctx._count(n)
     call("mt_intersect_primitives", ctx.handle, scene.handle, _ptr(rays), _ptr(isects), _ptr(count), n, mode)
     return rays, isects
 
@@ -366,7 +379,7 @@ def intersect_occlusion_records(ctx: Context, scene: Scene, rays, hits, count=No
     _need(rays, "rays", n, (RAY_RECORD_WORDS,))
     _need(hits, "hits", n, (), dtype="int32")
     if count is None:
-        count = ctx.scalar_i32(n)
+        count = ctx._count(n)
     call("mt_intersect_occlusion", ctx.handle, scene.handle, _ptr(rays), _ptr(hits), _ptr(count), n, mode)
     return hits
 
@@ -375,7 +388,7 @@ def shadow_rays(ctx: Context, o_tmin, d_tmax, prim, t, light_xyz, count=None):
     torch = _torch()
     n = o_tmin.shape[0]
     if count is None:
-        count = ctx.scalar_i32(n)
+        count = ctx._count(n)
     so = ctx.empty((n, 4), torch.float32)
     sd = ctx.empty((n, 4), torch.float32)
     valid = ctx.empty((n,), torch.int32)
@@ -481,9 +494,9 @@ def compact(ctx: Context, flags, flag_mode: int = 0, length=None, out_index=True
     torch = _torch()
     n = int(flags.shape[0])
     if length is None:
-        length = ctx.scalar_i32(n)
+        length = ctx._count(n)
     idx = ctx.empty((n,), torch.int32) if out_index else None
-    count = ctx.scalar_i32(0)
+    count = ctx._count(0)
     arr = (_lib.Payload * max(1, len(payloads)))()
     dsts = []
     for j, src in enumerate(payloads):

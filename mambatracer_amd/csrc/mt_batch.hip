@@ -805,7 +805,6 @@ extern "C" int32_t mt_batch_step(mt_batch* b, int32_t max_done, int64_t* done_ta
         MT_HIP_CHECK(hipStreamSynchronize(s));
         b->st.extension_rays = (int64_t)b->h_tot[0];
         b->st.shadow_rays = (int64_t)b->h_tot[1];
-        bool any = false;
         for (size_t i = 0; i < b->active_jobs.size();) {
             mt_batch::Job& J = b->active_jobs[i];
             if (!b->h_done[J.slot]) {
@@ -829,20 +828,9 @@ extern "C" int32_t mt_batch_step(mt_batch* b, int32_t max_done, int64_t* done_ta
             b->finished.push_back(J.d.tag);
             b->active_jobs.erase(b->active_jobs.begin() + (ptrdiff_t)i);
             b->active_dirty = true;
-            any = true;
         }
-        if (any) MT_HIP_CHECK(hipStreamSynchronize(s));
-        rc = mt_scan_check(b->ctx);
-        if (rc == MT_OK && b->gscratch) { // the captured compactions' workspace
-            mt_context* c = b->ctx;
-            void* sv = c->scratch;
-            const size_t svb = c->scratch_bytes;
-            c->scratch = b->gscratch;
-            c->scratch_bytes = b->gscratch_bytes;
-            rc = mt_scan_check(c);
-            c->scratch = sv;
-            c->scratch_bytes = svb;
-        }
+        // waits for the resolves; gscratch: the captured compactions' workspace
+        rc = mt_scan_check_with(b->ctx, b->gscratch);
         if (rc) return rc;
     }
     int nd = 0;

@@ -42,6 +42,7 @@ extern "C" int32_t mt_ctx_create(int32_t device, void* stream, int32_t flags, mt
     c->temp_bytes = 0;
     c->side = nullptr;
     c->nfj = 0;
+    c->host_words = nullptr;
     if (!(flags & MT_CTX_OWN_STREAM)) {
         c->stream = (hipStream_t)stream;
         c->own_stream = false;
@@ -74,9 +75,22 @@ extern "C" int32_t mt_ctx_destroy(mt_context* ctx)
         fe(hipEventDestroy(ctx->fork[k]));
         fe(hipEventDestroy(ctx->join[k]));
     }
+    if (ctx->host_words) fe(hipHostFree(ctx->host_words));
     if (ctx->own_stream) fe(hipStreamDestroy(ctx->stream));
     delete ctx;
     return fe.status("mt_ctx_destroy");
+}
+
+int32_t mt_ctx_host_words(mt_context* ctx, uint32_t** out)
+{
+    if (!ctx->host_words &&
+        hipHostMalloc(reinterpret_cast<void**>(&ctx->host_words), MT_HOST_WORDS * sizeof(uint32_t)) != hipSuccess) {
+        ctx->host_words = nullptr;
+        mt_set_error("cannot allocate pinned host memory");
+        return MT_ERR_ALLOC;
+    }
+    *out = ctx->host_words;
+    return MT_OK;
 }
 
 int32_t mt_ctx_side_stream(mt_context* ctx, hipStream_t* out)

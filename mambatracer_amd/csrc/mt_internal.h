@@ -73,7 +73,14 @@ struct mt_context {
     // every render reuses them
     hipEvent_t fork[64], join[64];
     int nfj;
+    // Pinned words that kernels write for the host to read after it has waited
+    // for the stream (first use allocates them): what a call reports takes
+    // one small launch and one wait, not a copy into pageable memory each.
+    uint32_t* host_words;
 };
+constexpr size_t MT_HOST_WORDS = 1024; // words 0..2: the look-back flags, from 16 on: a render's counts
+int32_t mt_ctx_host_words(mt_context* ctx, uint32_t** out);
+int32_t mt_scan_check_with(mt_context* ctx, void* more); // mt_scan_check with one more workspace
 
 // The context's side stream and its per-bounce fork / join events (created
 // on first use).

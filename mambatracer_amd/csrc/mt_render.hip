@@ -30,8 +30,6 @@
 #include "mt_path.h"
 #include "mt_traverse.h"
 
-#include <vector>
-
 namespace {
 
 constexpr int RT = 256; // threads per block
@@ -529,7 +527,7 @@ struct RenderPlan {
     char* base;
     size_t bytes;
     size_t oT, oL, oA_o, oA_d, oB_o, oB_d, oQA, oQB, oPrim, oT_, oAlive, oOcc, oSo, oSd, oSc, oCnt, oShc, oQsc,
-        oIlp, oTot, oSeed, oSlg, oHit, oHsc, oTail;
+        oIlp, oTot, oSeed, oSlg, oHit, oHsc, oTail, oZeroEnd;
     mt_lightgrid* grid; // guided environment mode: the grid the render samples and accumulates into
     bool fused; // camera rays traced in place, shadow adds fused, next queue appended by the shading stage
     int tail;   // fused loop: bounces tail..nb-1 run in one k_tail launch (0: the whole render; -1: none)
@@ -613,12 +611,14 @@ int32_t plan_render(const mt_scene* scene, const float* materials, const mt_envm
     R.oSo = take(16 * R.sq);
     R.oSd = take(16 * R.sq);
     R.oSc = take(16 * R.sq);
-    R.oCnt = take(4 * 64);
+    R.oHit = take(4 * R.sq);
+    R.oCnt = take(4 * 64); // from here to oZeroEnd: zeroed at the start of every render
+    R.oTail = take(4 * 2 * 64); // k_tail's live paths per bounce, then its shadow rays per bounce
     R.oShc = take(4 * 64 * (size_t)SHADOW_SEGS);
     R.oQsc = take(4 * 64 * (size_t)SHADOW_SEGS);
-    R.oHit = take(4 * R.sq);
     R.oHsc = take(4 * 64 * (size_t)SHADOW_SEGS);
-    R.oTail = take(4 * 2 * 64); // k_tail's live paths per bounce, then its shadow rays per bounce
+    R.oTot = take(8 * 8 * ILP_SLOTS);
+    R.oZeroEnd = bytes;
     R.want_ilp = (desc->flags & MT_RENDER_TRAVERSAL_STATS) != 0;
     R.fused = (desc->mode == MT_TRACE_PACKED || desc->mode == MT_TRACE_PACKED_STACK ||
                desc->mode == MT_TRACE_PACKED_SORTED || desc->mode == MT_TRACE_PACKED_POOL) && !R.want_ilp;
@@ -631,7 +631,6 @@ int32_t plan_render(const mt_scene* scene, const float* materials, const mt_envm
         !R.profile && R.np <= WHOLE_MAX)
         R.tail = 0;
     R.oIlp = R.want_ilp ? take(12 * (R.sq > n ? R.sq : n)) : 0;
-    R.oTot = take(8 * 8 * ILP_SLOTS);
     R.oSeed = take(4);
     R.oSlg = guided ? take(8 * R.sq) : 0;
     R.bytes = bytes;
@@ -764,12 +763,8 @@ int32_t enqueue_render(mt_context* ctx, RenderPlan& R)
         return MT_ERR_HIP;
     };
 
-    k_zero_i32<<<1, 64, 0, st>>>(counts, 64);
-    k_zero_i32<<<mt_blocks(64 * SHADOW_SEGS, RT), RT, 0, st>>>(shc, 64 * SHADOW_SEGS);
-    k_zero_i32<<<mt_blocks(64 * SHADOW_SEGS, RT), RT, 0, st>>>(qsc, 64 * SHADOW_SEGS);
-    k_zero_i32<<<mt_blocks(64 * SHADOW_SEGS, RT), RT, 0, st>>>(hsc, 64 * SHADOW_SEGS);
-    k_zero_i32<<<1, 128, 0, st>>>(I(R.oTail), 128);
-    k_zero_i32<<<mt_blocks(16 * ILP_SLOTS, RT), RT, 0, st>>>(reinterpret_cast<int*>(tot), 16 * ILP_SLOTS);
+    const int nzero = (int)((R.oZeroEnd - R.oCnt) / 4);
+    k_zero_i32<<<mt_blocks(nzero, RT), RT, 0, st>>>(counts, nzero);
     // Fused loop (default traversal, no traversal counters): bounce 0 traces
     // camera rays generated in place and shades with slot = pid; shadow rays
     // add their light inside the any-hit kernel; continuing paths append
@@ -919,62 +914,81 @@ int32_t enqueue_render(mt_context* ctx, RenderPlan& R)
     return rc;
 }
 
-// Reads the ray counts (and, when enabled, traversal counters and event
-// timings) of the last enqueued render; synchronises the stream.
-int32_t read_stats(mt_context* ctx, RenderPlan& R, mt_render_stats* stats)
+// What a render reports, in the context's pinned words.
+struct StatWords {
+    int live[64];   // paths entering each bounce
+    int shadow[64]; // shadow rays of each bounce
+    unsigned long long ilp[6];
+};
+
+// Block b sums bounce b's counts (the queue's length, or its segments' in the
+// fused loop from bounce 1 on, and k_tail's paths), the last block the
+// traversal counters.
+__global__ __launch_bounds__(256) void k_stats(const int* __restrict__ counts, const int* __restrict__ qsc,
+                                               const int* __restrict__ shc, const int* __restrict__ tail,
+                                               const unsigned long long* __restrict__ tot, int nb, int fused,
+                                               StatWords* __restrict__ out)
 {
-    hipStream_t st = ctx->stream;
-    const int nb = R.nb;
-    int hc[64];
-    std::vector<int> hs((size_t)nb * SHADOW_SEGS);
-    std::vector<unsigned long long> ht(8 * ILP_SLOTS);
-    hipError_t e = hipMemcpyAsync(hc, R.base + R.oCnt, sizeof(hc), hipMemcpyDeviceToHost, st);
-    if (e == hipSuccess) e = hipMemcpyAsync(hs.data(), R.base + R.oShc, hs.size() * sizeof(int), hipMemcpyDeviceToHost, st);
-    if (e == hipSuccess)
-        e = hipMemcpyAsync(ht.data(), R.base + R.oTot, ht.size() * sizeof(unsigned long long), hipMemcpyDeviceToHost,
-                           st);
-    if (e == hipSuccess) e = hipStreamSynchronize(st);
-    if (e != hipSuccess) {
-        mt_set_error("mt_render: stats readback failed: %s", hipGetErrorString(e));
-        return MT_ERR_HIP;
+    const int b = blockIdx.x;
+    if (b == nb) {
+        if (threadIdx.x < 6) {
+            unsigned long long v = 0;
+            for (int row = 0; row < ILP_SLOTS; row++) v += tot[8 * row + threadIdx.x];
+            out->ilp[threadIdx.x] = v;
+        }
+        return;
     }
+    __shared__ int s_sum[2];
+    if (threadIdx.x < 2) s_sum[threadIdx.x] = 0;
+    __syncthreads();
+    int q = 0, s = 0;
+    for (int p = threadIdx.x; p < SHADOW_SEGS; p += 256) {
+        q += qsc[b * SHADOW_SEGS + p];
+        s += shc[b * SHADOW_SEGS + p];
+    }
+    atomicAdd(&s_sum[0], q);
+    atomicAdd(&s_sum[1], s);
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        out->live[b] = (fused && b ? s_sum[0] : counts[b]) + tail[b];
+        out->shadow[b] = s_sum[1] + tail[64 + b];
+    }
+}
+
+// Enqueues the counts of the last enqueued render; *out holds them once the
+// stream has been waited for.
+int32_t enqueue_stats(mt_context* ctx, RenderPlan& R, const StatWords** out)
+{
+    uint32_t* words = nullptr;
+    const int32_t rc = mt_ctx_host_words(ctx, &words);
+    if (rc) return rc;
+    StatWords* w = reinterpret_cast<StatWords*>(words + 16);
+    static_assert(64 + sizeof(StatWords) <= MT_HOST_WORDS * sizeof(uint32_t), "pinned words");
+    auto I = [&](size_t off) { return reinterpret_cast<const int*>(R.base + off); };
+    k_stats<<<R.nb + 1, 256, 0, ctx->stream>>>(I(R.oCnt), I(R.oQsc), I(R.oShc), I(R.oTail),
+                                               reinterpret_cast<const unsigned long long*>(R.base + R.oTot), R.nb,
+                                               R.fused ? 1 : 0, w);
+    MT_LAUNCH_CHECK();
+    *out = w;
+    return MT_OK;
+}
+
+// The ray counts (and, when enabled, traversal counters and event timings) of
+// a render whose stream has been waited for.
+int32_t read_stats(const RenderPlan& R, const StatWords& w, mt_render_stats* stats)
+{
+    const int nb = R.nb;
     stats->extension_rays = 0;
     stats->shadow_rays = 0;
     stats->paths = R.np;
-    if (R.fused) { // bounces >= 1: the segment lengths of the appended queues
-        std::vector<int> hq((size_t)nb * SHADOW_SEGS);
-        e = hipMemcpyAsync(hq.data(), R.base + R.oQsc, hq.size() * sizeof(int), hipMemcpyDeviceToHost, st);
-        if (e == hipSuccess) e = hipStreamSynchronize(st);
-        if (e != hipSuccess) {
-            mt_set_error("mt_render: stats readback failed: %s", hipGetErrorString(e));
-            return MT_ERR_HIP;
-        }
-        for (int b = 1; b < nb; b++) {
-            int64_t c = 0;
-            for (int p = 0; p < SHADOW_SEGS; p++) c += hq[(size_t)b * SHADOW_SEGS + p];
-            hc[b] = (int)c;
-        }
+    for (int b = 0; b < 64; b++) {
+        stats->bounce_counts[b] = b < nb ? w.live[b] : 0;
+        stats->extension_rays += stats->bounce_counts[b];
+        if (b < nb) stats->shadow_rays += w.shadow[b];
     }
-    if (R.tail >= 0) { // k_tail's bounces: paths entering bounces > tail, shadow rays of bounces >= tail
-        int tl[128];
-        e = hipMemcpyAsync(tl, R.base + R.oTail, sizeof(tl), hipMemcpyDeviceToHost, st);
-        if (e == hipSuccess) e = hipStreamSynchronize(st);
-        if (e != hipSuccess) {
-            mt_set_error("mt_render: stats readback failed: %s", hipGetErrorString(e));
-            return MT_ERR_HIP;
-        }
-        for (int b = R.tail + 1; b < nb; b++) hc[b] += tl[b];
-        for (int b = R.tail; b < nb; b++) stats->shadow_rays += tl[64 + b];
-    }
-    for (int b = 0; b < 64; b++) stats->bounce_counts[b] = b < nb ? hc[b] : 0;
-    for (int b = 0; b < nb; b++) stats->extension_rays += hc[b];
-    for (int v : hs) stats->shadow_rays += v;
     for (int k = 0; k < 3; k++) {
-        stats->closest_ilp[k] = stats->any_ilp[k] = 0;
-        for (int row = 0; row < ILP_SLOTS; row++) {
-            stats->closest_ilp[k] += (int64_t)ht[8 * row + k];
-            stats->any_ilp[k] += (int64_t)ht[8 * row + 3 + k];
-        }
+        stats->closest_ilp[k] = (int64_t)w.ilp[k];
+        stats->any_ilp[k] = (int64_t)w.ilp[3 + k];
     }
     stats->closest_launches = stats->any_launches = 0;
     stats->closest_ms = stats->any_ms = 0.0f;
@@ -1008,14 +1022,12 @@ extern "C" int32_t mt_render(mt_context* ctx, const mt_scene* scene, const float
     if (rc) return rc;
     k_set_seed<<<1, 64, 0, ctx->stream>>>(seed_ptr(R), desc->seed);
     rc = enqueue_render(ctx, R);
-    if (rc == MT_OK && stats) rc = read_stats(ctx, R, stats);
-    const hipError_t se = hipStreamSynchronize(ctx->stream);
+    const StatWords* words = nullptr;
+    if (rc == MT_OK && stats) rc = enqueue_stats(ctx, R, &words);
+    if (rc == MT_OK) rc = mt_scan_check(ctx); // waits for the stream
+    else (void)hipStreamSynchronize(ctx->stream);
+    if (rc == MT_OK && stats) rc = read_stats(R, *words, stats);
     free_render(R);
-    if (rc == MT_OK && se != hipSuccess) {
-        mt_set_error("mt_render: %s", hipGetErrorString(se));
-        rc = MT_ERR_HIP;
-    }
-    if (rc == MT_OK) rc = mt_scan_check(ctx);
     return rc;
 }
 
@@ -1135,7 +1147,11 @@ extern "C" int32_t mt_render_graph_launch(mt_render_graph* g, uint32_t seed)
 extern "C" int32_t mt_render_graph_stats(mt_render_graph* g, mt_render_stats* stats)
 {
     MT_ARG_CHECK(g && stats, "mt_render_graph_stats: NULL argument");
-    int32_t rc = read_stats(g->ctx, g->R, stats);
+    const StatWords* words = nullptr;
+    int32_t rc = enqueue_stats(g->ctx, g->R, &words);
+    if (rc) return rc;
+    MT_HIP_CHECK(hipStreamSynchronize(g->ctx->stream));
+    rc = read_stats(g->R, *words, stats);
     if (rc) return rc;
     // the look-back error flag of the graph's own workspace (word 1)
     uint32_t flag = 0;

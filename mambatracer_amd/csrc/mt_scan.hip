@@ -575,27 +575,45 @@ extern "C" int32_t mt_compact_isects(mt_context* ctx, void* isects, int32_t* pix
     return MT_OK;
 }
 
-// Reports (and clears) the look-back spin-limit flag of the context.  A set
+// The look-back flags of up to three workspaces for the host (0 where there is none).
+__global__ void k_read_flags(const uint32_t* a, const uint32_t* b, const uint32_t* c, uint32_t* out)
+{
+    if (threadIdx.x == 0) {
+        out[0] = a ? a[1] : 0u;
+        out[1] = b ? b[1] : 0u;
+        out[2] = c ? c[1] : 0u;
+    }
+}
+
+// Reports (and clears) the look-back spin-limit flags of the context's
+// workspace, the device's no-alloc workspace and `more` (NULL: none).  A set
 // flag means a scan/compaction gave up waiting and its output is invalid.
+// Waits for the context's stream.
+int32_t mt_scan_check_with(mt_context* ctx, void* more)
+{
+    uint32_t* spaces[3] = {reinterpret_cast<uint32_t*>(ctx->scratch),
+                           reinterpret_cast<uint32_t*>(mt_noalloc_workspace(ctx->device)),
+                           reinterpret_cast<uint32_t*>(more)};
+    uint32_t* flags = nullptr;
+    int32_t rc = mt_ctx_host_words(ctx, &flags);
+    if (rc) return rc;
+    k_read_flags<<<1, 64, 0, ctx->stream>>>(spaces[0], spaces[1], spaces[2], flags);
+    MT_LAUNCH_CHECK();
+    MT_HIP_CHECK(hipStreamSynchronize(ctx->stream));
+    for (int k = 0; k < 3; k++) {
+        if (!flags[k]) continue;
+        rc = mt_buf_fill_i32(ctx, reinterpret_cast<int32_t*>(spaces[k] + 1), 0, 1);
+        if (rc) return rc;
+        mt_set_error("scan/compaction look-back exceeded its spin limit; results invalid");
+        return MT_ERR_STATE;
+    }
+    return MT_OK;
+}
+
 extern "C" int32_t mt_scan_check(mt_context* ctx)
 {
     MT_ARG_CHECK(ctx != nullptr, "mt_scan_check: ctx is NULL");
-    // the context's workspace, then the device's no-alloc workspace
-    void* spaces[2] = {ctx->scratch, mt_noalloc_workspace(ctx->device)};
-    for (void* sp : spaces) {
-        if (!sp) continue;
-        uint32_t flag = 0;
-        uint32_t* tk = reinterpret_cast<uint32_t*>(sp);
-        MT_HIP_CHECK(hipMemcpyAsync(&flag, tk + 1, sizeof(flag), hipMemcpyDeviceToHost, ctx->stream));
-        MT_HIP_CHECK(hipStreamSynchronize(ctx->stream));
-        if (flag) {
-            int32_t rc = mt_buf_fill_i32(ctx, reinterpret_cast<int32_t*>(tk + 1), 0, 1);
-            if (rc) return rc;
-            mt_set_error("scan/compaction look-back exceeded its spin limit; results invalid");
-            return MT_ERR_STATE;
-        }
-    }
-    return MT_OK;
+    return mt_scan_check_with(ctx, nullptr);
 }
 
 // identifyMeshLights + prefix sum + prepareLightInfo (LightConfiguration.cl:1-55).
