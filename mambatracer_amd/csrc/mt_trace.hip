@@ -235,8 +235,8 @@ __global__ __launch_bounds__(256, WaveLds<WT_STAGED>::WAVES) void k_trace_jobs(c
     __shared__ WaveLds<WT_STAGED> s_w[4];
     int count = *A.d_count;
     count = count < A.capacity ? count : A.capacity;
-    const int next = (int)(blockIdx.x * 4 + (threadIdx.x >> 6)) * A.run;
-    const int end = count < next + A.run ? count : next + A.run;
+    int next, end;
+    plain_run(count, WaveLds<WT_STAGED>::SLOTS, next, end);
     if (next >= end) return;
     wave_trace<false, true, WT_REFILL>(
         s_w, refs[tag[2 * next] >> shift], next, end,
@@ -1034,8 +1034,8 @@ int32_t mt_trace_jobs(mt_context* ctx, const MtSceneRef* refs, const int32_t* ta
     A.capacity = capacity;
     A.prim = prim;
     A.tout = t;
-    A.run = wave_run(capacity, WaveLds<WT_STAGED>::SLOTS);
-    k_trace_jobs<<<mt_blocks(capacity, 4 * A.run), 256, 0, ctx->stream>>>(refs, tag, shift, A);
+    k_trace_jobs<<<mt_blocks(wave_count(capacity, WaveLds<WT_STAGED>::SLOTS), 4), 256, 0, ctx->stream>>>(refs, tag, shift,
+                                                                                                   A);
     MT_LAUNCH_CHECK();
     return MT_OK;
 }
