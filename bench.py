@@ -580,8 +580,8 @@ def bench_c1(args) -> int:
         "other_lighting": others,
         "roofline": {
             "kernel": ("closest-hit traversal, packed layout: k_trace_camera (bounce 0, camera rays made in "
-                       f"place) and k_trace_pool (bounces 1-{(args.tail if tflags else job.max_bounces) - 1}, "
-                       "wave pools with lane refill), averaged over the job's launches"
+                       f"place) and k_trace_wave (bounces 1-{(args.tail if tflags else job.max_bounces) - 1}, "
+                       "waves that refill their lanes, nodes staged through LDS), averaged over the job's launches"
                        + (" (later bounces run inside k_tail)" if tflags else ""))
                       if job.mode == 0 else "closest-hit traversal (reference layout)",
             "bound": "hbm",
@@ -767,10 +767,11 @@ def bench_c2(args) -> int:
                                f"200-unit box), {n} rays uniform in the scene box, uniform directions; closest hit, "
                                "a shadow ray per ray to one light, any hit, stable compaction of the hit rays",
                    "rays": n, "traversal_layout": "packed",
-                   "traversal_modes": {k: {3: "short stack", 4: "persistent waves with per-lane refill",
-                                           6: "wave pools with lane refill",
+                   "traversal_modes": {k: {3: "waves that refill their lanes, each lane loading its node",
+                                           4: "the same, nodes staged through LDS by four lanes together",
+                                           6: "the same, nodes staged through LDS by four lanes together",
                                            7: "rays counting-sorted by origin cell (32^3 Morton), then "
-                                              "wave pools over that order"}.get(v, v)
+                                              "waves over that order, nodes staged through LDS"}.get(v, v)
                                        for k, v in modes.items()}},
         "stages_ms": {"closest": round(stage[0], 3), "shadow_setup": round(stage[1], 3),
                       "any": round(stage[2], 3), "compaction": round(stage[3], 4)},
@@ -779,8 +780,8 @@ def bench_c2(args) -> int:
         "compaction_GB_per_s": round(cbytes / stage[3] / 1e6, 1),
         "roofline": {
             "kernel": "closest-hit traversal (packed layout, "
-                      + {4: "k_trace_refill", 6: "k_trace_pool", 7: "k_bin_hist + k_bin_scatter + k_trace_pool"}
-                      .get(modes["closest"], "k_trace") + ")",
+                      + {7: "k_bin_hist + k_bin_scatter + k_trace_wave"}
+                      .get(modes["closest"], "k_trace_wave") + ")",
             "bound": "hbm",
             "achieved": round(traffic / (stage[0] / 1e3) / 1e9, 1) if traffic else None,
             "peak": HBM_PEAK_GBS,

@@ -961,10 +961,9 @@ class Batch:
         call("mt_batch_set_graphs", self.handle, 1 if on else 0)
 
     def set_trace_mode(self, mode: int) -> None:
-        """Closest-hit traversal of the shared queue: _lib.MT_TRACE_PACKED_STACK
-        (one ray per lane), _lib.MT_TRACE_PACKED_POOL (wave pools) or
-        _lib.MT_BATCH_TRACE_SPLIT (pools for the continuing paths, one ray per
-        lane for the new camera rays) (mt_batch_set_trace_mode)."""
+        """Closest-hit traversal of the shared queue: _lib.MT_TRACE_PACKED_STACK,
+        _lib.MT_TRACE_PACKED_POOL or _lib.MT_BATCH_TRACE_SPLIT, which all run
+        one kernel (mt_batch_set_trace_mode)."""
         call("mt_batch_set_trace_mode", self.handle, int(mode))
 
     def close(self) -> None:

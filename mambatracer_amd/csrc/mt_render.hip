@@ -25,6 +25,7 @@
 //      queue buffer (mt_compact; CCompact.execute in the reference).
 // With traversal counters or a non-default traversal layout the stages run
 // unfused (k_camera, mt_trace_any_seg, k_nee_accum): same paths, same bits.
+// A small render runs all of its bounces in one launch (k_tail).
 // After the last bounce the per-path radiance is averaged per pixel in a
 // fixed order, so the image is deterministic: no float atomics.
 #include "mt_path.h"
