@@ -55,6 +55,14 @@ extern "C" int32_t mt_ctx_create(int32_t device, void* stream, int32_t flags, mt
         }
         c->own_stream = true;
     }
+    // now: a later first use could meet another thread's capture
+    uint32_t* words = nullptr;
+    rc = mt_ctx_host_words(c, &words);
+    if (rc) {
+        if (c->own_stream) (void)hipStreamDestroy(c->stream);
+        delete c;
+        return rc;
+    }
     *out = c;
     return MT_OK;
 }

@@ -74,8 +74,8 @@ struct mt_context {
     hipEvent_t fork[64], join[64];
     int nfj;
     // Pinned words that kernels write for the host to read after it has waited
-    // for the stream (first use allocates them): what a call reports takes
-    // one small launch and one wait, not a copy into pageable memory each.
+    // for the stream: what a call reports takes one small launch and one wait,
+    // not a copy into pageable memory each.
     uint32_t* host_words;
 };
 constexpr size_t MT_HOST_WORDS = 1024; // words 0..2: the look-back flags, from 16 on: a render's counts
