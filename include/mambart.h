@@ -487,7 +487,7 @@ typedef struct {
     int32_t max_bounces;   /* path segments traced per sample (the reference fixes 15) */
     int32_t rr_start;      /* Russian roulette from this bounce on; < 0 disables */
     uint32_t seed;         /* job seed: RNG keys are (seed, path id, bounce, purpose) */
-    int32_t mode;          /* MT_TRACE_PACKED or MT_TRACE_REFERENCE traversal */
+    int32_t mode;          /* an MT_TRACE_ mode; _BINNED renders as _POOL (bounces are not sorted) */
     int32_t flags;         /* MT_RENDER_* bits */
 } mt_render_desc;
 

@@ -558,6 +558,11 @@ int32_t plan_render(const mt_scene* scene, const float* materials, const mt_envm
     R.np = (int)np64;
     R.nb = desc->max_bounces;
     R.desc = *desc;
+    // A bounce's rays are not sorted (mt_trace_closest_seg takes the mode as
+    // _POOL too), and mt_trace_closest's sort would take the context's
+    // workspace, which holds this render's state.
+    if (R.desc.mode == MT_TRACE_PACKED_BINNED) R.desc.mode = MT_TRACE_PACKED_POOL;
+    const int32_t mode = R.desc.mode;
     R.scene = scene;
     R.image = image;
     R.base = nullptr;
@@ -621,15 +626,15 @@ int32_t plan_render(const mt_scene* scene, const float* materials, const mt_envm
     R.oTot = take(8 * 8 * ILP_SLOTS);
     R.oZeroEnd = bytes;
     R.want_ilp = (desc->flags & MT_RENDER_TRAVERSAL_STATS) != 0;
-    R.fused = (desc->mode == MT_TRACE_PACKED || desc->mode == MT_TRACE_PACKED_STACK ||
-               desc->mode == MT_TRACE_PACKED_SORTED || desc->mode == MT_TRACE_PACKED_POOL) && !R.want_ilp;
+    R.fused = (mode == MT_TRACE_PACKED || mode == MT_TRACE_PACKED_STACK || mode == MT_TRACE_PACKED_SORTED ||
+               mode == MT_TRACE_PACKED_POOL) && !R.want_ilp;
     R.tail = (desc->flags >> MT_RENDER_TAIL_SHIFT) & 63;
     R.profile = (desc->flags & MT_RENDER_PROFILE) != 0;
     if (!R.fused || R.tail == 0 || R.tail >= R.nb) R.tail = -1; // the tail applies to the fused loop's bounces >= 1
     // a small render of the default traversal: all bounces in one launch (the
     // profile's per-stage times need the stages)
-    if (R.tail < 0 && R.fused && (desc->mode == MT_TRACE_PACKED || desc->mode == MT_TRACE_PACKED_STACK) &&
-        !R.profile && R.np <= WHOLE_MAX)
+    if (R.tail < 0 && R.fused && (mode == MT_TRACE_PACKED || mode == MT_TRACE_PACKED_STACK) && !R.profile &&
+        R.np <= WHOLE_MAX)
         R.tail = 0;
     R.oIlp = R.want_ilp ? take(12 * (R.sq > n ? R.sq : n)) : 0;
     R.oSeed = take(4);
