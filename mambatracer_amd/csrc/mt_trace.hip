@@ -49,7 +49,7 @@ struct TraceArgs {
     int* occluded;
     int* stats;
     int plain;    // mt_scene::plain
-    int run;      // rays per wave over a plain queue
+    int run;      // rays per wave over a binned order
     MtSegQueue seg; // segmented queue (seg.counts set) instead of *d_count
     const int* order; // binned traversal: entry k is ray order[k], its results go there (null: ray k)
 };
@@ -109,9 +109,9 @@ __global__ __launch_bounds__(256) void k_trace(TraceArgs A)
 }
 
 // Wave traversal (wave_trace) of a queue: each wave owns a run of consecutive
-// entries (segmented queue: an even share of its segment, seg_run; over a
-// binned order, work-groups in per-XCD runs) and refills its finished lanes
-// from it.
+// entries (plain queue: a share of the live entries, plain_run; segmented
+// queue: an even share of its segment, seg_run; over a binned order,
+// work-groups in per-XCD runs) and refills its finished lanes from it.
 template <bool ANY, bool WIDE, WaveForm F>
 __global__ __launch_bounds__(256, WaveLds<F>::WAVES) void k_trace_wave(TraceArgs A)
 {
@@ -123,16 +123,19 @@ __global__ __launch_bounds__(256, WaveLds<F>::WAVES) void k_trace_wave(TraceArgs
         int count = *A.d_count;
         count = count < A.capacity ? count : A.capacity;
         count = count > 0 ? count : 0;
-        // over a binned order, consecutive entries start in the same cell and
-        // walk the same subtrees: the groups that hold entries are numbered
-        // in per-XCD runs (the grid is sized for the capacity; the rest leave
-        // at once below)
-        const unsigned used = (unsigned)(((int64_t)count + 4 * A.run - 1) / (4 * A.run));
-        const unsigned g = A.order && blockIdx.x < used ? xcd_chunked_group(blockIdx.x, used, XCD_RUN) : blockIdx.x;
-        const int64_t first = ((int64_t)g * 4 + (threadIdx.x >> 6)) * A.run;
-        if (first >= count) return;
-        next = (int)first;
-        end = count - next < A.run ? count : next + A.run;
+        if (A.order) {
+            // consecutive entries start in the same cell and walk the same
+            // subtrees: the groups that hold entries are numbered in per-XCD
+            // runs (the grid is sized for the capacity; the rest leave at once)
+            const unsigned used = (unsigned)(((int64_t)count + 4 * A.run - 1) / (4 * A.run));
+            const unsigned g = blockIdx.x < used ? xcd_chunked_group(blockIdx.x, used, XCD_RUN) : blockIdx.x;
+            const int64_t first = ((int64_t)g * 4 + (threadIdx.x >> 6)) * A.run;
+            if (first >= count) return;
+            next = (int)first;
+            end = count - next < A.run ? count : next + A.run;
+        } else {
+            plain_run(count, WaveLds<F>::SLOTS, next, end);
+        }
     }
     if (next >= end) return;
     wave_trace<ANY, WIDE, WT_REFILL>(
@@ -459,9 +462,10 @@ int32_t launch_trace(mt_context* ctx, const mt_scene* sc, const float* o_tmin,
         kern = wide ? k_trace_wave<ANY, true, WT_STAGED_DEEP> : k_trace_wave<ANY, false, WT_STAGED_DEEP>;
         slots = WaveLds<WT_STAGED_DEEP>::SLOTS;
     }
-    A.run = A.order ? WT_BINNED_RUN : wave_run(capacity, slots);
+    A.run = WT_BINNED_RUN;
+    const int64_t waves = A.order ? (capacity + (int64_t)A.run - 1) / A.run : wave_count(capacity, slots);
     const int64_t groups = seg.counts ? (int64_t)seg.nseg * wave_seg_groups(seg.seg_cap, seg.nseg, slots)
-                                      : (capacity + 4 * (int64_t)A.run - 1) / (4 * (int64_t)A.run);
+                                      : (waves + 3) / 4;
     kern<<<dim3((unsigned)groups), block, 0, s>>>(A);
     MT_LAUNCH_CHECK();
     return MT_OK;
@@ -727,9 +731,9 @@ __device__ __forceinline__ void record_result(const TraceArgs& A, const float4* 
     iw[20] = 1; // hit = HIT_MARKER
 }
 
-// The packed layout: each wave traces a run of slots (wave_trace); LAYOUT 1
-// and 2 below trace one slot per lane over the reference arrays or without a
-// stack.
+// The packed layout: each wave traces a run of the live slots (plain_run), and
+// the whole grid marks the slots past *d_count as misses; LAYOUT 1 and 2 below
+// trace one slot per lane over the reference arrays or without a stack.
 template <bool WIDE>
 __global__ __launch_bounds__(256, WaveLds<WT_DIRECT>::WAVES) void k_intersect_records_wave(TraceArgs A, const float4* __restrict__ normals,
                                                                            const float2* __restrict__ uvs,
@@ -739,14 +743,11 @@ __global__ __launch_bounds__(256, WaveLds<WT_DIRECT>::WAVES) void k_intersect_re
     int count = *A.d_count;
     count = count < A.capacity ? count : A.capacity;
     count = count > 0 ? count : 0;
-    const int64_t first = ((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * A.run;
-    if (first >= A.capacity) return;
-    const int next = (int)first;
-    const int stop = A.capacity - next < A.run ? A.capacity : next + A.run;
-    // slots past *d_count are misses
-    for (int id = (next > count ? next : count) + (int)__lane_id(); id < stop; id += 64)
-        record_result(A, normals, uvs, rays, isects, id, -1, 0.0f);
-    const int end = count < stop ? count : stop;
+    for (int64_t id = count + (int64_t)blockIdx.x * blockDim.x + threadIdx.x; id < A.capacity;
+         id += (int64_t)gridDim.x * blockDim.x)
+        record_result(A, normals, uvs, rays, isects, (int)id, -1, 0.0f);
+    int next, end;
+    plain_run(count, WaveLds<WT_DIRECT>::SLOTS, next, end);
     if (next >= end) return;
     wave_trace<false, WIDE, WT_REFILL>(
         s_w, MtSceneRef{A.pn, A.pt, A.root, A.plain}, next, end,
@@ -784,10 +785,10 @@ __global__ __launch_bounds__(256, WaveLds<WT_DIRECT>::WAVES) void k_occlusion_re
     __shared__ WaveLds<WT_DIRECT> s_w[4];
     int count = *A.d_count;
     count = count < A.capacity ? count : A.capacity;
-    const int64_t first = ((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * A.run;
-    if (first >= count) return;
-    const int next = (int)first;
-    const int end = count - next < A.run ? count : next + A.run;
+    count = count > 0 ? count : 0;
+    int next, end;
+    plain_run(count, WaveLds<WT_DIRECT>::SLOTS, next, end);
+    if (next >= end) return;
     wave_trace<true, WIDE, WT_REFILL>(
         s_w, MtSceneRef{A.pn, A.pt, A.root, A.plain}, next, end,
         [&](int id, RayT& r, MtSceneRef&) { record_ray(rays + 5 * (size_t)id, r); },
@@ -1087,12 +1088,11 @@ extern "C" int32_t mt_intersect_primitives(mt_context* ctx, const mt_scene* sc, 
     dim3 grid(mt_blocks(capacity, 256)), block(256);
     hipStream_t s = ctx->stream;
     // every other packed mode gives the same bits: one kernel
-    A.run = wave_run(capacity, WaveLds<WT_DIRECT>::SLOTS);
-    const int waves = mt_blocks(capacity, 4 * A.run);
+    const int groups = mt_blocks(wave_count(capacity, WaveLds<WT_DIRECT>::SLOTS), 4);
     if (mode == MT_TRACE_REFERENCE) k_intersect_records<1><<<grid, block, 0, s>>>(A, nrm, uvs, R, I);
     else if (mode == MT_TRACE_PACKED_NO_STACK) k_intersect_records<2><<<grid, block, 0, s>>>(A, nrm, uvs, R, I);
-    else if (scene_wide(sc)) k_intersect_records_wave<true><<<waves, block, 0, s>>>(A, nrm, uvs, R, I);
-    else k_intersect_records_wave<false><<<waves, block, 0, s>>>(A, nrm, uvs, R, I);
+    else if (scene_wide(sc)) k_intersect_records_wave<true><<<groups, block, 0, s>>>(A, nrm, uvs, R, I);
+    else k_intersect_records_wave<false><<<groups, block, 0, s>>>(A, nrm, uvs, R, I);
     MT_LAUNCH_CHECK();
     return MT_OK;
 }
@@ -1120,11 +1120,11 @@ extern "C" int32_t mt_intersect_occlusion(mt_context* ctx, const mt_scene* sc, c
     const float4* R = reinterpret_cast<const float4*>(rays);
     dim3 grid(mt_blocks(capacity, 256)), block(256);
     hipStream_t s = ctx->stream;
-    A.run = wave_run(capacity, WaveLds<WT_DIRECT>::SLOTS);
+    const int groups = mt_blocks(wave_count(capacity, WaveLds<WT_DIRECT>::SLOTS), 4);
     if (mode == MT_TRACE_REFERENCE) k_occlusion_records<1><<<grid, block, 0, s>>>(A, R, hits);
     else if (mode == MT_TRACE_PACKED_NO_STACK) k_occlusion_records<2><<<grid, block, 0, s>>>(A, R, hits);
-    else if (scene_wide(sc)) k_occlusion_records_wave<true><<<mt_blocks(capacity, 4 * A.run), block, 0, s>>>(A, R, hits);
-    else k_occlusion_records_wave<false><<<mt_blocks(capacity, 4 * A.run), block, 0, s>>>(A, R, hits);
+    else if (scene_wide(sc)) k_occlusion_records_wave<true><<<groups, block, 0, s>>>(A, R, hits);
+    else k_occlusion_records_wave<false><<<groups, block, 0, s>>>(A, R, hits);
     MT_LAUNCH_CHECK();
     return MT_OK;
 }
