@@ -342,14 +342,20 @@ constexpr int WT_BINNED_RUN = 512;       // rays per wave of a sorted batch: nei
 
 enum WaveForm { WT_DIRECT, WT_STAGED, WT_STAGED_DEEP };
 
+// Aligned for the 16-byte loads into `node` and the 8-byte reads of it, wherever
+// the compiler places a kernel's LDS objects.
 template <WaveForm F>
-struct WaveLds {
+struct alignas(16) WaveLds {
     static constexpr int ROWS = F == WT_DIRECT ? 12 : F == WT_STAGED ? 9 : 14; // pending subtrees per lane
     static constexpr int WAVES = F == WT_DIRECT ? 8 : F == WT_STAGED ? 6 : 5;  // per SIMD
     static constexpr int SLOTS = 1024 * WAVES; // waves that the GPU's 1024 SIMDs hold at once
     char node[F == WT_DIRECT ? 256 : 4 * WT_SLOT]; // direct: only the row under the stack, which idle lanes read
     int stack[ROWS + 1][64];                       // row 0: WT_NONE under the bottom
 };
+template <WaveForm F>
+constexpr bool wave_lds_aligned = alignof(WaveLds<F>) == 16 && offsetof(WaveLds<F>, node) == 0 && WT_SLOT % 16 == 0;
+static_assert(wave_lds_aligned<WT_DIRECT> && wave_lds_aligned<WT_STAGED> && wave_lds_aligned<WT_STAGED_DEEP>,
+              "load slots on 16 bytes");
 typedef __attribute__((address_space(3))) char lds_char;
 typedef __attribute__((address_space(3))) int lds_int;
 typedef float vf2 __attribute__((ext_vector_type(2)));
