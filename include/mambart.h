@@ -709,10 +709,13 @@ int32_t mt_batch_set_iterations(mt_batch* batch, int32_t iterations);
  * Synchronises the context. */
 int32_t mt_batch_set_graphs(mt_batch* batch, int32_t on);
 /* Closest-hit traversal of the engine's shared queue (no counterpart in the
- * reference): MT_BATCH_TRACE_SPLIT (= MT_TRACE_PACKED, the default),
- * MT_TRACE_PACKED_STACK or MT_TRACE_PACKED_POOL.  All of them run one kernel
- * now (staged nodes; each lane takes its slot's scene with its ray); the call
- * is kept for its callers.  Images do not depend on it.  Synchronises the
+ * reference), each lane with its slot's scene: MT_BATCH_TRACE_SPLIT
+ * (= MT_TRACE_PACKED, the default: nodes staged through LDS),
+ * MT_TRACE_PACKED_STACK (each lane loads its own nodes: about 1% faster where
+ * most rays are coherent, 2-11% slower elsewhere) or MT_TRACE_PACKED_POOL
+ * (staged with a deeper stack and fewer waves: up to 5% faster for small
+ * queues or deep trees, up to 4% slower elsewhere).  Images do not depend on
+ * it.  The serving autotuner tries them per workload.  Synchronises the
  * context. */
 #define MT_BATCH_TRACE_SPLIT 8
 int32_t mt_batch_set_trace_mode(mt_batch* batch, int32_t mode);

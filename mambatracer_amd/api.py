@@ -961,9 +961,10 @@ class Batch:
         call("mt_batch_set_graphs", self.handle, 1 if on else 0)
 
     def set_trace_mode(self, mode: int) -> None:
-        """Closest-hit traversal of the shared queue: _lib.MT_TRACE_PACKED_STACK,
-        _lib.MT_TRACE_PACKED_POOL or _lib.MT_BATCH_TRACE_SPLIT, which all run
-        one kernel (mt_batch_set_trace_mode)."""
+        """Closest-hit traversal of the shared queue: _lib.MT_BATCH_TRACE_SPLIT
+        (the default, nodes staged through LDS), _lib.MT_TRACE_PACKED_POOL (the
+        same with a deeper stack) or _lib.MT_TRACE_PACKED_STACK (each lane loads
+        its nodes) (mt_batch_set_trace_mode)."""
         call("mt_batch_set_trace_mode", self.handle, int(mode))
 
     def close(self) -> None:

@@ -230,16 +230,17 @@ __global__ __launch_bounds__(256) void k_trace_sorted(TraceArgs A)
 // Rays of many jobs in one queue: ray id's scene is refs[tag[2*id] >> shift]
 // (the job word of a wavefront slot); a lane takes its ray's scene with the
 // ray, so a ray's result does not depend on which queue carries it.
-// Staged: 24 uneven soup jobs 23.4 -> 15.4 ms (direct 17.0).
-__global__ __launch_bounds__(256, WaveLds<WT_STAGED>::WAVES) void k_trace_jobs(const MtSceneRef* __restrict__ refs,
-                                                                              const int* __restrict__ tag, int shift,
-                                                                              TraceArgs A)
+template <WaveForm F>
+__global__ __launch_bounds__(256, WaveLds<F>::WAVES) void k_trace_jobs(const MtSceneRef* __restrict__ refs,
+                                                                      const int* __restrict__ tag, int shift,
+                                                                      TraceArgs A)
 {
-    __shared__ WaveLds<WT_STAGED> s_w[4];
+    __shared__ WaveLds<F> s_w[4];
     int count = *A.d_count;
     count = count < A.capacity ? count : A.capacity;
+    count = count > 0 ? count : 0;
     int next, end;
-    plain_run(count, WaveLds<WT_STAGED>::SLOTS, next, end);
+    plain_run(count, WaveLds<F>::SLOTS, next, end);
     if (next >= end) return;
     wave_trace<false, true, WT_REFILL>(
         s_w, refs[tag[2 * next] >> shift], next, end,
@@ -1025,7 +1026,7 @@ int32_t mt_trace_any_seg(mt_context* ctx, const mt_scene* scene, const float4* o
 
 int32_t mt_trace_jobs(mt_context* ctx, const MtSceneRef* refs, const int32_t* tag, int32_t shift,
                       const float4* o_tmin, const float4* d_tmax, const int32_t* d_count, int32_t capacity,
-                      int32_t* prim, float* t)
+                      int32_t* prim, float* t, int32_t mode)
 {
     if (capacity == 0) return MT_OK;
     TraceArgs A{};
@@ -1035,8 +1036,20 @@ int32_t mt_trace_jobs(mt_context* ctx, const MtSceneRef* refs, const int32_t* ta
     A.capacity = capacity;
     A.prim = prim;
     A.tout = t;
-    k_trace_jobs<<<mt_blocks(wave_count(capacity, WaveLds<WT_STAGED>::SLOTS), 4), 256, 0, ctx->stream>>>(refs, tag, shift,
-                                                                                                   A);
+    // Three forms of the walk (WaveForm), by the caller's choice.  ms for 24 soup
+    // jobs / 12 and 24 of 400K-1.5M triangles / 16 jobs on open spheres / 6 jobs
+    // through a queue of 256K paths: staged 20.9, 16.8, 31.9, 8.69, 13.0; direct
+    // 22.7, 17.6, 35.4, 8.60, 13.3; deep 21.5, 16.7, 31.8, 8.77, 12.3.
+    auto kern = k_trace_jobs<WT_STAGED>;
+    int slots = WaveLds<WT_STAGED>::SLOTS;
+    if (mode == MT_TRACE_PACKED_STACK) {
+        kern = k_trace_jobs<WT_DIRECT>;
+        slots = WaveLds<WT_DIRECT>::SLOTS;
+    } else if (mode == MT_TRACE_PACKED_POOL) {
+        kern = k_trace_jobs<WT_STAGED_DEEP>;
+        slots = WaveLds<WT_STAGED_DEEP>::SLOTS;
+    }
+    kern<<<mt_blocks(wave_count(capacity, slots), 4), 256, 0, ctx->stream>>>(refs, tag, shift, A);
     MT_LAUNCH_CHECK();
     return MT_OK;
 }

@@ -271,13 +271,14 @@ def autotune_batch(ctx: api.Context, requests: List[Request], arena_bytes: int =
                    trace_modes=None, graphs=(True, False), objective: str = "jobs_per_s"):
     """Chooses the multi-job engine's settings for a workload: the queue
     capacity (paths in flight per iteration), the bounce iterations per host
-    round trip, the closest-hit traversal of the shared queue (the engine's
-    modes run one kernel) and graph replay.  `requests` is a sample of the
+    round trip, the closest-hit traversal of the shared queue (nodes staged
+    through LDS, loaded by each lane, or staged with a deep stack) and graph
+    replay.  `requests` is a sample of the
     workload (its scenes, sizes and sample counts), served through
     serve_batched per trial: objective "jobs_per_s" submits them at once and
     the setting with the most jobs/s wins; "p99" keeps their arrival times
     and the lowest p99 latency wins.  Coordinate search from (largest capacity, 8 iterations, the
-    split traversal, graphs): each dimension in turn takes its best value with
+    default traversal, graphs): each dimension in turn takes its best value with
     the others held.  Every setting renders the same images.  Returns (best
     setting, [(setting, jobs/s or p99 ms), ...])."""
     from . import _lib
