@@ -27,6 +27,11 @@ struct v3 {
     float x, y, z;
 };
 
+__device__ __forceinline__ uint32_t lane_rank(uint64_t mask)
+{ // set bits of `mask` below this lane (v_mbcnt_lo/hi)
+    return __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
+}
+
 __device__ __forceinline__ v3 mk3(float x, float y, float z) { return v3{x, y, z}; }
 __device__ __forceinline__ v3 add3(v3 a, v3 b) { return mk3(a.x + b.x, a.y + b.y, a.z + b.z); }
 __device__ __forceinline__ v3 sub3(v3 a, v3 b) { return mk3(a.x - b.x, a.y - b.y, a.z - b.z); }

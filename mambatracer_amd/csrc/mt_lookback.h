@@ -2,6 +2,7 @@
 // (mt_scan.hip, described there) and the BVH builder's fused flag scan
 // (mt_bvh.hip).
 #pragma once
+#include "mt_devmath.h"
 #include "mt_internal.h"
 
 namespace {
@@ -20,11 +21,6 @@ __device__ __forceinline__ uint64_t pack_status(uint32_t epoch, uint32_t flag, u
 }
 
 __device__ __forceinline__ int lane_id() { return __lane_id(); }
-
-__device__ __forceinline__ uint32_t lane_rank(uint64_t mask)
-{ // number of set bits of `mask` below this lane (v_mbcnt_lo/hi)
-    return __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
-}
 
 // Decoupled look-back by wave 0 of the tile.  Returns the exclusive prefix of
 // `tile` (all lanes of wave 0 agree); publishes the tile's inclusive prefix.

@@ -106,15 +106,6 @@ __host__ __device__ inline void path_pixel(int pid, int w, int h, int spp, int& 
     y = band * 8 + (r - x * rows);
 }
 
-// First path id of pixel (x, y) (its samples follow it).
-__host__ __device__ inline int pixel_first_path(int x, int y, int w, int h, int spp)
-{
-    const int band = y >> 3, full_bands = h >> 3;
-    const int k = band < full_bands ? band * 8 * w + x * 8 + (y & 7)
-                                    : full_bands * 8 * w + x * (h - 8 * full_bands) + (y - 8 * band);
-    return k * spp;
-}
-
 // Primary ray of path `pid` (pixel from path_pixel), jittered inside its
 // pixel; tMin 0.001 and tMax inf as initGlobalRay (Util.cl:577-587).
 __device__ __forceinline__ void camera_ray(const Camera& C, int pid, uint32_t seed, float4& o_tmin,
@@ -434,7 +425,7 @@ __device__ __forceinline__ int wave_append(bool flag, int* counter)
         if (__lane_id() == 0) base = atomicAdd(counter, (int)__popcll(m));
         base = __shfl(base, 0);
     }
-    return base + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+    return base + (int)lane_rank(m);
 }
 
 // Shadow-ray and path queues are segmented (see MtSegQueue): work-group b of
@@ -457,17 +448,6 @@ inline int shadow_seg_cap(int64_t slots, int group)
 {
     const int64_t groups = (slots + group - 1) / group;
     return (int)((groups + NSEG - 1) / NSEG) * group;
-}
-
-// Entry of this lane in a segmented queue walked chunk-major: work-group b
-// takes chunk b / SHADOW_SEGS of segment b % SHADOW_SEGS (seg_cap is a
-// multiple of the group size), so the live chunks at the front of every
-// segment are dispatched first.
-template <int NSEG = SHADOW_SEGS>
-__device__ __forceinline__ int seg_entry(int seg_cap)
-{
-    const int p = blockIdx.x % NSEG, c = blockIdx.x / NSEG;
-    return p * seg_cap + c * blockDim.x + threadIdx.x;
 }
 
 // Whether entry `id` of a segmented queue of NSEG segments holds an item.

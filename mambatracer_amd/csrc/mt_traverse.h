@@ -240,11 +240,6 @@ __device__ __forceinline__ bool parent_walk(const float4* __restrict__ pn, const
     return true;
 }
 
-__device__ __forceinline__ uint32_t lane_rank(uint64_t mask)
-{ // set bits of `mask` below this lane (v_mbcnt_lo/hi)
-    return __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
-}
-
 // Work-groups go to the 8 XCDs in turn (group b on XCD b mod 8), each XCD
 // with its own L2.  Where neighbouring work-groups trace rays that walk the
 // same subtrees, renumbering the groups so that each XCD takes runs of
