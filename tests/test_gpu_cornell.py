@@ -72,7 +72,9 @@ def test_cornell_mesh_parses_as_the_fixture(cornell):
     np.testing.assert_array_equal(faces[:, 9] & 0xFFFF, want)
 
 
-@pytest.mark.parametrize("flags", [0, _lib.MT_RENDER_PICKED_LIGHT])
+# A render this small runs in one launch; MT_RENDER_PROFILE keeps the launches per bounce.
+@pytest.mark.parametrize("flags", [0, _lib.MT_RENDER_PICKED_LIGHT, _lib.MT_RENDER_PROFILE,
+                                   _lib.MT_RENDER_PICKED_LIGHT | _lib.MT_RENDER_PROFILE])
 def test_cornell_render_matches_oracle(ctx, cornell, flags):
     print(f"[case] cornell box flags={flags}", flush=True)
     fx, points, normals, faces, nodes, bounds, depth, _ = cornell

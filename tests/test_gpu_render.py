@@ -50,9 +50,11 @@ def _render_both(ctx, c1_small, job, with_env=True):
     return img.cpu().numpy()[:, :3], st, oimg, rays
 
 
-def test_render_matches_oracle(ctx, c1_small):
-    print("[case] render c1 small", flush=True)
-    job = W.RenderJob(width=160, height=90, spp=4, pos=(0.0, 0.5, -8.0), look=(0.0, -1.0, 0.0))
+# A render this small runs in one launch; MT_RENDER_PROFILE keeps the launches per bounce.
+@pytest.mark.parametrize("flags", [0, _lib.MT_RENDER_PROFILE])
+def test_render_matches_oracle(ctx, c1_small, flags):
+    print(f"[case] render c1 small flags={flags}", flush=True)
+    job = W.RenderJob(width=160, height=90, spp=4, pos=(0.0, 0.5, -8.0), look=(0.0, -1.0, 0.0), flags=flags)
     img, st, oimg, rays = _render_both(ctx, c1_small, job)
     ext, sh = int(st.extension_rays), int(st.shadow_rays)
     print(f"gpu rays {ext}+{sh}, oracle {rays[0]}+{rays[1]}")
@@ -61,7 +63,8 @@ def test_render_matches_oracle(ctx, c1_small):
     assert np.isfinite(img).all() and img.mean() > 0
 
 
-@pytest.mark.parametrize("flags", [0, _lib.MT_RENDER_PICKED_LIGHT])
+@pytest.mark.parametrize("flags", [0, _lib.MT_RENDER_PICKED_LIGHT, _lib.MT_RENDER_PROFILE,
+                                   _lib.MT_RENDER_PICKED_LIGHT | _lib.MT_RENDER_PROFILE])
 def test_render_mesh_lights_matches_oracle(ctx, c1_small, flags):
     """Emitter hits (LightHitPass emitter branch) and DirectLight on area
     lights picked from the mesh-light list, beside the environment."""
@@ -132,7 +135,9 @@ def test_render_stats_counters(ctx, c1_small):
 @pytest.mark.parametrize("mesh_lights", [False, True])
 def test_fused_and_staged_loops_agree(ctx, c1_small, mesh_lights):
     """The default loop fuses the camera pass into bounce 0's traversal and
-    the direct-light add into the any-hit kernel; with traversal counters on,
+    the direct-light add into the any-hit kernel (a render this small then runs
+    in one launch unless MT_RENDER_PROFILE or another mode keeps the launches
+    per bounce); with traversal counters on,
     or another traversal layout, every stage is a separate launch.  Same
     paths, so images, ray counts and per-bounce counts are bit-identical."""
     print(f"[case] fused vs staged loop, mesh lights {mesh_lights}", flush=True)
@@ -150,13 +155,16 @@ def test_fused_and_staged_loops_agree(ctx, c1_small, mesh_lights):
     env = api.CEnvironment(ctx)
     env.setEnvironmentMap(W.env_map())
     base = dict(width=100, height=60, spp=3, pos=(0.0, 0.5, -8.0), look=(0.0, -1.0, 0.0), seed=5)
-    runs = [W.RenderJob(**base),                                           # fused
+    runs = [W.RenderJob(**base),                                           # one launch
+            W.RenderJob(**base, flags=_lib.MT_RENDER_PROFILE),             # fused, launches per bounce
             W.RenderJob(**base, mode=_lib.MT_TRACE_PACKED_SORTED),         # fused, direction-sorted lanes
             W.RenderJob(**base, mode=_lib.MT_TRACE_PACKED_POOL),           # fused, wave-pool lanes
             W.RenderJob(**base, flags=_lib.MT_RENDER_TAIL_FROM(1)),        # fused, bounces 1.. in one launch
             W.RenderJob(**base, flags=_lib.MT_RENDER_TAIL_FROM(3)),        # fused, bounces 3.. in one launch
             W.RenderJob(**base, flags=_lib.MT_RENDER_TAIL_FROM(W.RenderJob().max_bounces - 1)),  # last bounce only
             W.RenderJob(**base, flags=_lib.MT_RENDER_TAIL_FROM(W.RenderJob().max_bounces)),      # past the end: off
+            W.RenderJob(**base, flags=_lib.MT_RENDER_TAIL_FROM(W.RenderJob().max_bounces)
+                        | _lib.MT_RENDER_PROFILE),                         # past the end, launches per bounce
             W.RenderJob(**base, mode=_lib.MT_TRACE_PACKED_POOL,            # wave pools, then the tail
                         flags=_lib.MT_RENDER_TAIL_FROM(2)),
             W.RenderJob(**base, flags=_lib.MT_RENDER_TRAVERSAL_STATS),     # staged, same traversal
@@ -177,7 +185,8 @@ def test_tail_with_many_live_paths(ctx, mesh_lights):
     into the late bounces (a fifth at bounce 3, against 0.2% in the open
     config-1 scene), so the one-launch tail carries thousands of paths per
     segment sweep and refills every lane many times.  Tail from bounce 1, 3
-    and 6 against the per-bounce launches: same image bits, ray counts and
+    and 6, and the whole render in one launch (no tail asked for), against the
+    per-bounce launches (MT_RENDER_PROFILE): same image bits, ray counts and
     per-bounce counts."""
     print(f"[case] tail on a soup, mesh lights {mesh_lights}", flush=True)
     points, faces, nodes, bounds, depth = W.soup_scene(200_000, 61)
@@ -196,8 +205,8 @@ def test_tail_with_many_live_paths(ctx, mesh_lights):
     env.setEnvironmentMap(W.env_map())
     job = W.soup_job(W.JobSpec(0, 0, 128, 4, 6100 + int(mesh_lights)))
     out = []
-    for tail in (0, 1, 3, job.max_bounces - 2):
-        job.flags = _lib.MT_RENDER_TAIL_FROM(tail)
+    for tail in (None, 0, 1, 3, job.max_bounces - 2):
+        job.flags = _lib.MT_RENDER_PROFILE if tail is None else _lib.MT_RENDER_TAIL_FROM(tail)
         img, st = api.render(ctx, sc, dm, env, job, light_faces=lf, num_lights=nl)
         out.append((img.cpu().numpy(), st))
     ref_img, ref_st = out[0]
@@ -214,9 +223,10 @@ def test_tail_with_many_live_paths(ctx, mesh_lights):
 
 @pytest.mark.parametrize("w,h,spp", [(1, 1, 1), (7, 3, 5), (17, 9, 1)])
 def test_tiny_jobs_fused_and_staged_agree(ctx, c1_small, w, h, spp):
-    """Jobs far smaller than one work-group or one queue segment: the fused
-    loop (appended, segmented path queues) and the staged loop (compaction)
-    give the same image bits and ray counts, and the counts add up."""
+    """Jobs far smaller than one work-group or one queue segment: one launch,
+    the fused loop (MT_RENDER_PROFILE: appended, segmented path queues) and the
+    staged loop (compaction) give the same image bits and ray counts, and the
+    counts add up."""
     print(f"[case] tiny job {w}x{h}x{spp}", flush=True)
     points, normals, faces, nodes, bounds, depth = c1_small
     sc = api.Scene(ctx, points, faces, nodes, bounds, depth, normals=normals)
@@ -224,10 +234,10 @@ def test_tiny_jobs_fused_and_staged_agree(ctx, c1_small, w, h, spp):
     env = api.CEnvironment(ctx)
     env.setEnvironmentMap(W.env_map())
     base = dict(width=w, height=h, spp=spp, pos=(0.0, 0.5, -8.0), look=(0.0, -1.0, 0.0), seed=9)
-    (img_f, st_f), (img_s, st_s), (img_t, st_t) = [
-        api.render(ctx, sc, dm, env, W.RenderJob(**base, **extra))
-        for extra in ({}, {"flags": _lib.MT_RENDER_TRAVERSAL_STATS}, {"flags": _lib.MT_RENDER_TAIL_FROM(1)})]
-    for img, st in ((img_s, st_s), (img_t, st_t)):
+    (img_f, st_f), *rest = [
+        api.render(ctx, sc, dm, env, W.RenderJob(**base, flags=flags))
+        for flags in (_lib.MT_RENDER_PROFILE, 0, _lib.MT_RENDER_TRAVERSAL_STATS, _lib.MT_RENDER_TAIL_FROM(1))]
+    for img, st in rest:
         np.testing.assert_array_equal(img_f.cpu().numpy().view(np.int32), img.cpu().numpy().view(np.int32))
         assert list(st_f.bounce_counts) == list(st.bounce_counts)
         assert int(st_f.shadow_rays) == int(st.shadow_rays)

@@ -2,7 +2,9 @@
 HIP graph and replayed per frame.  Bar: every replay's image and ray counts
 equal mt_render's for the same seed bit for bit (the graph replays the same
 launches), with eager library work and synchronisations between replays, and
-one replay against the oracle's restatement at the render tolerance."""
+one replay against the oracle's restatement at the render tolerance.  Renders
+this small capture their one launch; the loop with its side stream is captured
+in test_gpu_render_overlap.py and, with traversal counters, here."""
 import numpy as np
 import pytest
 import torch

@@ -56,11 +56,13 @@ def _diff(name, a, b):
     return n
 
 
-@pytest.mark.parametrize("tile_pdf,tail", [(False, 0), (True, 0), (False, 2), (True, 1)])
+@pytest.mark.parametrize("tile_pdf,tail", [(False, 0), (True, 0), (False, 2), (True, 1), (False, None), (True, None)])
 def test_guided_frames_match_oracle(ctx, c1_small, tile_pdf, tail):
-    """tail > 0: bounces tail.. run in one k_tail launch (MT_RENDER_TAIL_FROM)."""
+    """tail > 0: bounces tail.. run in one k_tail launch (MT_RENDER_TAIL_FROM);
+    0: all of them do, a render this small; None: launches per bounce
+    (MT_RENDER_PROFILE)."""
     flags = _lib.MT_RENDER_LIGHTGRID_ENV | (_lib.MT_RENDER_LIGHTGRID_TILE_PDF if tile_pdf else 0)
-    flags |= _lib.MT_RENDER_TAIL_FROM(tail)
+    flags |= _lib.MT_RENDER_PROFILE if tail is None else _lib.MT_RENDER_TAIL_FROM(tail)
     job = W.RenderJob(width=96, height=54, spp=4, max_bounces=6, pos=(0.0, 0.5, -8.0), look=(0.0, -1.0, 0.0),
                       flags=flags)
     print(f"[case] guided frames tile_pdf={tile_pdf} tail={tail}", flush=True)
@@ -109,7 +111,9 @@ def test_guided_flags_need_a_grid(ctx, c1_small):
 def test_guided_render_graph_replays_match_render(ctx, c1_small, tail):
     """A captured guided render replays the same image and grid sums as
     mt_render from the same grid state (eager work between replays); with
-    tail > 0 the capture holds the one-launch tail (MT_RENDER_TAIL_FROM)."""
+    tail > 0 the capture holds the one-launch tail (MT_RENDER_TAIL_FROM), with
+    0 the whole render as one launch (larger captures:
+    test_gpu_render_overlap.py)."""
     print(f"[case] guided render graph tail={tail}", flush=True)
     job = W.RenderJob(width=64, height=40, spp=2, max_bounces=5, pos=(0.0, 0.5, -8.0), look=(0.0, -1.0, 0.0),
                       flags=_lib.MT_RENDER_LIGHTGRID_ENV | _lib.MT_RENDER_LIGHTGRID_TILE_PDF

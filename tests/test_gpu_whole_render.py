@@ -3,8 +3,8 @@ keeps the launches per bounce.  Both against each other, and the late-bounce
 launch with few lanes per wave, at the numbers of paths where the lanes per
 wave change (4096 waves of 2, 4 .. 64 lanes) and where the one launch ends.
 Bar: the image's bits, the ray counts and the paths per bounce are the same
-(the per-bounce loop is compared with the oracle in test_gpu_render.py, whose
-small jobs also run as one launch)."""
+(both are compared with the oracle in test_gpu_render.py, the per-bounce loop
+with its side stream in test_gpu_render_overlap.py)."""
 import numpy as np
 import pytest
 
