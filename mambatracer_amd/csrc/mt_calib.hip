@@ -19,8 +19,10 @@
  *           fminf/fmaxf (24)
  *   kind 3  8 v_add_u32 + 8 v_xor_b32 (16)
  *   kind 4  8 v_cmp_f32 + 8 v_cndmask_b32 + 8 v_add_f32, a select per
- *           chain as the traversal's branch-free code makes them (24)
- *   kind 5  16 v_fma_f32 (16)
+ *           chain as the traversal's branch-free code makes them (24): the
+ *           interleaved add hides most of what compares and selects cost in a row
+ *   kind 5  16 v_fma_f32 with a scalar-register multiplicand (16): the scalar
+ *           source makes it a 4-cycle instruction, as it does an add
  *   kind 6  8 correctly rounded divisions, 11 instructions each: 2
  *           v_div_scale_f32, v_rcp_f32, 5 FMA, v_mul_f32, v_div_fmas_f32,
  *           v_div_fixup_f32 (88)

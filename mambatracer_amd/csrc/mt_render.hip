@@ -353,8 +353,8 @@ constexpr int TAIL_SLOTS = 1024 * TAIL_WAVES; // waves that the GPU's 1024 SIMDs
 // its slowest ray) against it: 14400 soup paths 1078 -> 617 us, 16384 on open
 // spheres 502 -> 250, 4096 in a closed room 1305 -> 733, 131072 there 1773 ->
 // 1592, 262144 in the soup 3211 -> 2346, 240000 on spheres 696 -> 397.  Past
-// one round of lanes it loses: 524288 soup paths 3999 -> 3911, 993K 4.82 ->
-// 9.9 ms.
+// one round of lanes the gain goes (524288 soup paths 3999 -> 3911) and then
+// turns (993K 4.82 -> 9.9 ms).
 constexpr int WHOLE_MAX = 64 * TAIL_SLOTS;
 template <bool WIDE, bool WHOLE>
 __global__ __launch_bounds__(RT, TAIL_WAVES) void k_tail(ShadeArgs A, MtSceneRef scene, int np, int nb, int lanes,

@@ -286,12 +286,18 @@ __device__ __forceinline__ unsigned seg_sweep_group()
 // Wave traversal: one ray per lane of a wave, every ray in the reference's
 // visiting order (the packed layout of trace_packed below).
 //
-// What bounds it on gfx950: vector issue and the vector L1.  Measured rates
-// per wave64 instruction and SIMD: 2.4 cycles for f32 add / mul, moves, integer
-// add and logic; 4.2-4.5 for compares, selects, min / max (also of three),
-// DPP and shift-adds.  The L1 looks one 64-byte piece up per cycle, and four
-// 16-byte loads of a node by lanes that hold different nodes are four pieces
-// per lane.  So:
+// What bounds it on gfx950: the vector memory path and vector issue between
+// them, with latency in the gaps; neither is full by itself.  Per wave64
+// instruction and SIMD, f32 add / mul / FMA, moves, integer add and logic take
+// 2.1-2.4 cycles; compares, selects, min / max (also of three), DPP, shift-adds
+// and whatever reads a scalar register 4.1, unless they alternate with the
+// first kind (max + add: 4.2 the pair).  The L1 looks one 64-byte piece up per
+// cycle, and four 16-byte loads of a node by lanes that hold different nodes
+// are four pieces per lane.  Measured per CU: camera rays (direct) 3.9 cycles
+// per VALU instruction and SIMD, 0.81 pieces per cycle, the data return busy
+// 0.86 of the time; bounces (staged) 7.5, 0.46, 0.89 and LDS 0.21 (0.09 of it
+// bank conflicts); a sorted random batch (staged, deep) 6.3, 0.55, 0.93, 0.22.
+// So:
 //  * a lane's pending subtrees are a plain stack of references in LDS (one
 //    write and one read per step, both unconditional) instead of a register
 //    queue moved on every push and pop and a 128-bit bitstack; entries past
