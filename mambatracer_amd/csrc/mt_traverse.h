@@ -659,20 +659,20 @@ __device__ __forceinline__ int leaf_prim(const float4* __restrict__ pt, int chil
 // its lanes together need, but a wave of few lanes costs the SIMD as much as
 // a full one (with launch and read-back, 4096 camera rays in waves of 16: 278
 // us, of 4: 251; 30000 in waves of 16: 303, of 4: 391).
-__host__ __device__ inline int wave_run(int64_t n, int slots)
+__host__ __device__ inline int wave_run(int n, int slots)
 {
-    const int64_t r = (n / slots + 15) & ~(int64_t)15, few = (n / 2048 + 4) & ~(int64_t)3;
-    if (r <= WT_MIN_RUN) return (int)(few < WT_MIN_RUN ? few : WT_MIN_RUN);
-    return (int)(r > WT_MAX_RUN ? WT_MAX_RUN : r);
+    const int r = (n / slots + 15) & ~15, few = (n / 2048 + 4) & ~3;
+    if (r <= WT_MIN_RUN) return few < WT_MIN_RUN ? few : WT_MIN_RUN;
+    return r > WT_MAX_RUN ? WT_MAX_RUN : r;
 }
 
 // Waves of a launch over a plain queue of up to n entries whose length only the
 // device knows: as many as a full queue takes, and enough to fill the slots
 // with fewer entries.
-inline int64_t wave_count(int64_t n, int slots)
+inline int64_t wave_count(int n, int slots)
 {
-    const int64_t full = (n + wave_run(n, slots) - 1) / wave_run(n, slots);
-    const int64_t few = (n + WT_MIN_RUN - 1) / WT_MIN_RUN;
+    const int64_t full = ((int64_t)n + wave_run(n, slots) - 1) / wave_run(n, slots);
+    const int64_t few = ((int64_t)n + WT_MIN_RUN - 1) / WT_MIN_RUN;
     const int64_t fill = few < slots ? few : slots;
     return full > fill ? full : fill;
 }
@@ -685,12 +685,12 @@ inline int64_t wave_count(int64_t n, int slots)
 // 557, 380 -> 383, what a queue of that capacity takes).
 __device__ __forceinline__ void plain_run(int count, int slots, int& next, int& end)
 {
-    const int64_t waves = (int64_t)gridDim.x * 4;
-    int64_t run = wave_run(count, slots);
-    if (run * waves < count) run = (count + waves - 1) / waves; // the grid covers the queue
-    const int64_t first = ((int64_t)blockIdx.x * 4 + (int)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6)) * run;
+    const unsigned waves = gridDim.x * 4; // at most 2^31 / 4 (wave_count)
+    int run = wave_run(count, slots);
+    if ((int64_t)run * waves < count) run = (int)(((unsigned)count + waves - 1) / waves); // the grid covers the queue
+    const int64_t first = (int64_t)(blockIdx.x * 4 + (int)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6)) * run;
     next = first < count ? (int)first : count;
-    end = count - next < run ? count : next + (int)run;
+    end = count - next < run ? count : next + run;
 }
 
 // Work-groups per segment of a queue of nseg segments.
